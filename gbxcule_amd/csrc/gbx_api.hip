@@ -38,7 +38,7 @@ struct gbx_ctx {
   // and a masked restore skips them.
   bool dead_rows_dirty = false;
   std::vector<uint8_t> boot_host;  // the power-on fill of rows 0x00-0xFF
-  uint64_t* hash_k = nullptr;
+  HashTable hash{};
   int dbg[4] = {0, 0, 0, 0};
 };
 
@@ -70,7 +70,30 @@ uint64_t splitmix(uint64_t i) {
   return z ^ (z >> 31);
 }
 
-constexpr int kHashLen = kMemSize + 128;
+// Weights of the state hash (HashTable) on the host, computed once.
+struct HashHost {
+  std::vector<int8_t> digits = std::vector<int8_t>(kHashDigits, 0);
+  std::vector<uint64_t> fields = std::vector<uint64_t>(64 + kCartStateStride);
+  uint64_t bias = 0;
+  HashHost() {
+    for (uint32_t a = 0; a < (uint32_t)kMemSize; ++a) {
+      uint64_t k = splitmix(a);
+      bias += 128u * k;
+      // address 64 c + 4 i + q is byte i of lanes 16 q + column of chunk c
+      int8_t* d = &digits[((size_t)(a >> 6) * 64u + (a & 3u) * 16u) * 16u + ((a >> 2) & 15u)];
+      for (uint32_t j = 0; j < 8; ++j) {
+        const int64_t v = (int64_t)(int8_t)(k & 0xFFu);  // -128..127; a carry past the last digit is mod 2^64
+        d[j * 16u] = (int8_t)v;
+        k = (k - (uint64_t)v) >> 8;
+      }
+    }
+    for (size_t i = 0; i < fields.size(); ++i) fields[i] = splitmix((uint64_t)kMemSize + i);
+  }
+};
+const HashHost& hash_host() {
+  static const HashHost h;
+  return h;
+}
 
 // Device address of `scratch` per device, taken once per device with that
 // device current (gbx_create) and kept for the life of the process.
@@ -114,7 +137,7 @@ void free_ctx(gbx_ctx* c) {
   void* ptrs[] = {s.mem, s.cram, s.cs, s.sc, s.cnt, s.serial, s.actions, s.obs, s.reward,
                   s.pix, s.pix_packed, s.latches, s.frame_bg, (void*)s.rom, (void*)s.boot, (void*)s.recs,
                   c->snap.mem, c->snap.cram, c->snap.serial, c->snap.pix, c->snap.cs,
-                  c->snap.sc, c->snap.cnt, c->hash_k};
+                  c->snap.sc, c->snap.cnt, c->hash.digits, c->hash.fields};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   delete c;
@@ -275,20 +298,22 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   A(dalloc(&c->snap.cs, (size_t)kCartStateStride));
   A(dalloc(&c->snap.sc, (size_t)kNumFields));
   A(dalloc(&c->snap.cnt, (size_t)2));
-  A(dalloc(&c->hash_k, (size_t)kHashLen));
+  A(dalloc(&c->hash.digits, kHashDigits));
+  A(dalloc(&c->hash.fields, (size_t)(64 + kCartStateStride)));
   if (e != hipSuccess) {
     free_ctx(c);
     return fail(GBX_E_HIP, std::string("device allocation failed: ") + hipGetErrorString(e));
   }
-  std::vector<uint64_t> k(kHashLen);
-  for (int i = 0; i < kHashLen; ++i) k[i] = splitmix((uint64_t)i);
   const std::vector<Rec> recs = build_records(rom, rom_bytes, boot);
   A(hipMemcpy(drom, rom, (size_t)rom_bytes, hipMemcpyHostToDevice));
   A(hipMemcpy(drom + rom_bytes, boot, 0x100, hipMemcpyHostToDevice));
   A(hipMemset(drom + rom_bytes + 0x100, 0xFF, (size_t)kOpenBusBytes));
   A(hipMemcpy(dboot, boot, 0x100, hipMemcpyHostToDevice));
   A(hipMemcpy(drecs, recs.data(), recs.size() * sizeof(Rec), hipMemcpyHostToDevice));
-  A(hipMemcpy(c->hash_k, k.data(), k.size() * 8, hipMemcpyHostToDevice));
+  const HashHost& hh = hash_host();
+  A(hipMemcpy(c->hash.digits, hh.digits.data(), hh.digits.size(), hipMemcpyHostToDevice));
+  A(hipMemcpy(c->hash.fields, hh.fields.data(), hh.fields.size() * 8, hipMemcpyHostToDevice));
+  c->hash.bias = hh.bias;
   if (e != hipSuccess) {
     free_ctx(c);
     return fail(GBX_E_HIP, std::string("upload failed: ") + hipGetErrorString(e));
@@ -432,7 +457,7 @@ int gbx_write_mem(gbx_ctx* ctx, int32_t env_lo, int32_t env_hi, int32_t lo, int3
 int gbx_state_hash(gbx_ctx* ctx, uint64_t* out_dev, void* stream) {
   CHECK_CTX(ctx);
   if (!out_dev) return fail(GBX_E_INVALID, "out is NULL");
-  HIP_TRY(launch_hash(ctx->s, ctx->hash_k, out_dev, (hipStream_t)stream));
+  HIP_TRY(launch_hash(ctx->s, ctx->hash, out_dev, (hipStream_t)stream));
   return GBX_OK;
 }
 

@@ -39,7 +39,16 @@ hipError_t launch_masked_reset(const DevState& s, const SnapState& snap, const u
                                int live, hipStream_t st);
 hipError_t launch_gather(const DevState& s, const uint16_t* addrs, int k, uint8_t* out,
                          hipStream_t st);
-hipError_t launch_hash(const DevState& s, const uint64_t* K, uint64_t* out, hipStream_t st);
+// Weights of the state hash: balanced base-256 digits of the memory weights in
+// hash_mem_kernel's operand order, the weights of the scalar fields and the
+// cartridge state, and 128 times the sum of the memory weights.
+struct HashTable {
+  int8_t* digits;    // [65536 / 64][64 lanes][16]
+  uint64_t* fields;  // [64 + kCartStateStride]
+  uint64_t bias;
+};
+constexpr size_t kHashDigits = (size_t)kMemSize * 16;
+hipError_t launch_hash(const DevState& s, const HashTable& k, uint64_t* out, hipStream_t st);
 // buf[count][len] env-major <-> memory of envs [env_lo, env_lo + count),
 // addresses [lo, lo + len); to_image = 0 reads the image into buf, 1 writes
 // buf into the image.  The caller checks the ranges.

@@ -834,24 +834,88 @@ __global__ void gather_kernel(DevState s, const uint16_t* addrs, int k, uint8_t*
 // Per-env linear hash: sum of byte * K[addr] over memory, plus the scalar
 // fields, counters and cartridge state weighted by further K entries
 // (wrapping uint64 arithmetic; K = splitmix64(index)).
-__global__ void hash_kernel(DevState s, const uint64_t* K, uint64_t* out) {
+//
+// hash_state_kernel writes the scalar part and the bias below; the memory
+// part, a [envs x 65536] by [65536 x 8] product of bytes and base-256 digits
+// of K, is added by hash_mem_kernel on the matrix cores.  Digits are balanced
+// (-128..127) and bytes are taken as byte - 128, so that both are signed
+// 8-bit operands; `bias` is 128 times the sum of K over memory.  Partial sums
+// are whole numbers below 2^30, so the result is exact.
+__global__ void hash_state_kernel(DevState s, const uint64_t* K, uint64_t bias, uint64_t* out) {
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (uint32_t)s.n) return;
-  const uint8_t* mb = s.mem + ((size_t)block_of(e) << 22);
-  const uint32_t lane = e & (kEnvBlock - 1);
-  uint64_t h = 0;
-  for (uint32_t a = 0; a < (uint32_t)kMemSize; ++a)
-    h += (uint64_t)mb[((size_t)a << kEnvBlockShift) | lane] * K[a];
+  uint64_t h = bias;
   for (int f = 0; f < kNumFields; ++f) {
     if (f == F_INSTR || f == F_CYCLES) continue;
     const int32_t v = f == F_ACTIONS ? s.actions[e] : s.sc[sc_index(e, f)];
-    h += (uint64_t)(uint32_t)v * K[kMemSize + f];
+    h += (uint64_t)(uint32_t)v * K[f];
   }
-  h += (uint64_t)s.cnt[cnt_index(e, 0)] * K[kMemSize + F_INSTR];
-  h += (uint64_t)s.cnt[cnt_index(e, 1)] * K[kMemSize + F_CYCLES];
+  h += (uint64_t)s.cnt[cnt_index(e, 0)] * K[F_INSTR];
+  h += (uint64_t)s.cnt[cnt_index(e, 1)] * K[F_CYCLES];
   for (int k = 0; k < kCartStateStride; ++k)
-    h += (uint64_t)(uint32_t)s.cs[cs_index(e, k)] * K[kMemSize + 64 + k];
+    h += (uint64_t)(uint32_t)s.cs[cs_index(e, k)] * K[64 + k];
   out[e] = h;
+}
+
+// One 64-byte address row holds one byte of each env of a block.  A wavefront
+// takes 64 addresses of a block at a time: load i reads rows 4i..4i+3 (256
+// contiguous bytes), so lane l holds, for envs 4(l % 16)..+3, the bytes of
+// addresses 4i + l / 16, i = 0..15.  Sixteen 4x4 byte transposes in registers
+// turn them into the A operands of four 16x16x64 products, one per env of the
+// lane's four (row = l % 16, depth l / 16 by i); the B operand is the digit
+// table in the same depth order (kHashDigits bytes, columns 8-15 zero).
+// Bound by HBM: 64 KiB per env, and one digit-table load (1 KiB, L2) per 4 KiB
+// of memory.  At 4,096 envs 42 us, 6.3 TB/s of memory read; one lane per env
+// walking its 65,536 bytes in turn took 5,680 us (16 workgroups on the chip).
+typedef int v4i __attribute__((ext_vector_type(4)));
+constexpr int kHashWaves = 4;
+__device__ __forceinline__ void transpose4(uint32_t& a, uint32_t& b, uint32_t& c, uint32_t& d) {
+  const uint32_t ab0 = __builtin_amdgcn_perm(b, a, 0x05010400u), ab1 = __builtin_amdgcn_perm(b, a, 0x07030602u);
+  const uint32_t cd0 = __builtin_amdgcn_perm(d, c, 0x05010400u), cd1 = __builtin_amdgcn_perm(d, c, 0x07030602u);
+  a = __builtin_amdgcn_perm(cd0, ab0, 0x05040100u);
+  b = __builtin_amdgcn_perm(cd0, ab0, 0x07060302u);
+  c = __builtin_amdgcn_perm(cd1, ab1, 0x05040100u);
+  d = __builtin_amdgcn_perm(cd1, ab1, 0x07060302u);
+}
+__global__ __launch_bounds__(64 * kHashWaves) void hash_mem_kernel(DevState s, const v4i* digits, uint32_t chunks,
+                                                                   uint64_t* out) {
+  __shared__ unsigned long long sum[kEnvBlock];
+  const uint32_t t = threadIdx.x, l = t & 63u;
+  const uint32_t w = __builtin_amdgcn_readfirstlane(t >> 6);
+  if (t < (uint32_t)kEnvBlock) sum[t] = 0;
+  __syncthreads();
+  const uint8_t* mb = s.mem + ((size_t)blockIdx.x << 22) + (l << 2);
+  v4i acc[4] = {};
+  const uint32_t c0 = blockIdx.y * chunks;
+  for (uint32_t c = c0 + w; c < c0 + chunks; c += kHashWaves) {
+    const v4i kd = digits[(size_t)c * 64u + l];
+    uint32_t r[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      r[i] = __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(mb + ((size_t)c << 12) + i * 256));
+#pragma unroll
+    for (int i = 0; i < 16; i += 4) transpose4(r[i], r[i + 1], r[i + 2], r[i + 3]);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      // byte - 128 as a signed byte is the byte with bit 7 flipped
+      const v4i a = {(int)(r[j] ^ 0x80808080u), (int)(r[4 + j] ^ 0x80808080u), (int)(r[8 + j] ^ 0x80808080u),
+                     (int)(r[12 + j] ^ 0x80808080u)};
+      acc[j] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, kd, acc[j], 0, 0, 0);
+    }
+  }
+  // lane l holds digit column l % 16 of rows 4 (l / 16) + k
+  if ((l & 15u) < 8u) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int k = 0; k < 4; ++k)
+        atomicAdd(&sum[4u * (4u * (l >> 4) + (uint32_t)k) + (uint32_t)j],
+                  (unsigned long long)(int64_t)acc[j][k] << (8u * (l & 7u)));
+  }
+  __syncthreads();
+  const uint32_t e = blockIdx.x * kEnvBlock + t;
+  if (t < (uint32_t)kEnvBlock && e < (uint32_t)s.n)
+    atomicAdd(reinterpret_cast<unsigned long long*>(out) + e, sum[t]);
 }
 
 // Layout converters for the synchronous export/import helpers.
@@ -1023,9 +1087,17 @@ hipError_t launch_gather(const DevState& s, const uint16_t* addrs, int k, uint8_
   return hipGetLastError();
 }
 
-hipError_t launch_hash(const DevState& s, const uint64_t* K, uint64_t* out, hipStream_t st) {
+hipError_t launch_hash(const DevState& s, const HashTable& k, uint64_t* out, hipStream_t st) {
   if (s.n <= 0) return hipSuccess;
-  hipLaunchKernelGGL(hash_kernel, dim3((unsigned)((s.n + 255) / 256)), dim3(256), 0, st, s, K, out);
+  hipLaunchKernelGGL(hash_state_kernel, dim3((unsigned)((s.n + 255) / 256)), dim3(256), 0, st, s, k.fields, k.bias, out);
+  // Below 2,048 workgroups (8 per CU) a block's addresses are split among
+  // several, each adding its part to the envs' sums, so that few envs fill
+  // the chip too; at 64 parts a wavefront is down to four chunks.
+  const int blocks = s.npad / kEnvBlock;
+  int parts = 1;
+  while (parts < 64 && blocks * parts < 2048) parts <<= 1;
+  hipLaunchKernelGGL(hash_mem_kernel, dim3((unsigned)blocks, (unsigned)parts), dim3(64 * kHashWaves), 0, st, s,
+                     reinterpret_cast<const v4i*>(k.digits), (uint32_t)(kMemSize / 64 / parts), out);
   return hipGetLastError();
 }
 

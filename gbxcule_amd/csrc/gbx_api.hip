@@ -135,7 +135,7 @@ bool differs_from_fill(const gbx_ctx* c, int32_t addr, const uint8_t* bytes, int
 void free_ctx(gbx_ctx* c) {
   DevState& s = c->s;
   void* ptrs[] = {s.mem, s.cram, s.cs, s.sc, s.cnt, s.serial, s.actions, s.obs, s.reward,
-                  s.pix, s.pix_packed, s.latches, s.frame_bg, (void*)s.rom, (void*)s.boot, (void*)s.recs,
+                  s.pix, s.pix_packed, s.latches, s.frame_bg, (void*)s.rom, (void*)s.boot, (void*)s.recs, (void*)s.fused,
                   c->snap.mem, c->snap.cram, c->snap.serial, c->snap.pix, c->snap.cs,
                   c->snap.sc, c->snap.cnt, c->hash.digits, c->hash.fields};
   for (void* p : ptrs)
@@ -151,33 +151,6 @@ hipError_t dalloc(T** p, size_t count) {
 // The ROM buffer is the ROM, then the boot image, then one 16 KiB window of
 // 0xFF that an unmapped ROM bank reads (open bus).
 constexpr int64_t kOpenBusBytes = 0x4000;
-
-// Pre-decoded instruction records for the step kernel's fetch: one 512-bit
-// record (gbx_decode.h) per byte of the ROM buffer, built from that byte and
-// the next two bytes of the same image.  Bytes past the end of an image read
-// as 0; the kernel only uses a record when all three instruction bytes lie
-// inside one 16 KiB ROM window or inside the boot image.
-std::vector<Rec> build_records(const uint8_t* rom, int64_t rom_bytes, const uint8_t* boot) {
-  std::vector<Rec> r((size_t)(rom_bytes + 0x100 + kOpenBusBytes));
-  auto fill = [&](const uint8_t* img, int64_t len, size_t base) {
-    for (int64_t i = 0; i < len; ++i) {
-      const uint32_t op = img[i], b1 = i + 1 < len ? img[i + 1] : 0u,
-                     b2 = i + 2 < len ? img[i + 2] : 0u;
-      r[base + (size_t)i] = decode_insn(op, b1, b2);
-    }
-  };
-  fill(rom, rom_bytes, 0);
-  // LY poll loops and block-copy loops whose bytes lie inside one 16 KiB window
-  for (int64_t i = 0; i + 5 < rom_bytes; ++i) {
-    const uint32_t pl = poll_loop_len(rom + i, (uint32_t)std::min<int64_t>(8, rom_bytes - i));
-    if (pl != 0u && (i & 0x3FFF) + pl <= 0x4000) r[(size_t)i] = mark_poll_loop(r[(size_t)i], rom + i);
-    if ((i & 0x3FFF) <= 0x3FF8 && i + 7 < rom_bytes && copy_loop_at(rom + i)) r[(size_t)i] = mark_copy_loop(r[(size_t)i]);
-  }
-  fill(boot, 0x100, (size_t)rom_bytes);
-  const std::vector<uint8_t> ff(kOpenBusBytes, 0xFF);
-  fill(ff.data(), kOpenBusBytes, (size_t)rom_bytes + 0x100);
-  return r;
-}
 
 // Header parse (reference core/cartridge.py:139-187).
 int parse_header(const uint8_t* rom, int64_t rom_len, int* kind, int64_t* rom_bytes,
@@ -285,12 +258,15 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   A(dalloc(&s.frame_bg, (size_t)kScreenW * kScreenH));
   uint8_t *drom = nullptr, *dboot = nullptr;
   Rec* drecs = nullptr;
+  Fused* dfused = nullptr;
   A(dalloc(&drom, (size_t)(rom_bytes + 0x100 + kOpenBusBytes)));
   A(dalloc(&dboot, (size_t)0x100));
   A(dalloc(&drecs, (size_t)(rom_bytes + 0x100 + kOpenBusBytes)));
+  A(dalloc(&dfused, (size_t)(rom_bytes + 0x100 + kOpenBusBytes)));
   s.rom = drom;
   s.boot = dboot;
   s.recs = reinterpret_cast<const uint4*>(drecs);
+  s.fused = reinterpret_cast<const uint4*>(dfused);
   A(dalloc(&c->snap.mem, (size_t)kMemSize));
   A(dalloc(&c->snap.cram, (size_t)s.cram_stride));
   A(dalloc(&c->snap.serial, (size_t)kSerialMax));
@@ -304,12 +280,11 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
     free_ctx(c);
     return fail(GBX_E_HIP, std::string("device allocation failed: ") + hipGetErrorString(e));
   }
-  const std::vector<Rec> recs = build_records(rom, rom_bytes, boot);
   A(hipMemcpy(drom, rom, (size_t)rom_bytes, hipMemcpyHostToDevice));
   A(hipMemcpy(drom + rom_bytes, boot, 0x100, hipMemcpyHostToDevice));
   A(hipMemset(drom + rom_bytes + 0x100, 0xFF, (size_t)kOpenBusBytes));
   A(hipMemcpy(dboot, boot, 0x100, hipMemcpyHostToDevice));
-  A(hipMemcpy(drecs, recs.data(), recs.size() * sizeof(Rec), hipMemcpyHostToDevice));
+  A(launch_build_records(s, rom_bytes + 0x100 + kOpenBusBytes, nullptr));
   const HashHost& hh = hash_host();
   A(hipMemcpy(c->hash.digits, hh.digits.data(), hh.digits.size(), hipMemcpyHostToDevice));
   A(hipMemcpy(c->hash.fields, hh.fields.data(), hh.fields.size() * 8, hipMemcpyHostToDevice));

@@ -526,4 +526,88 @@ __host__ __device__ constexpr Rec decode_insn(uint32_t op, uint32_t b1, uint32_t
   return bind_bytes(decode_base(op == 0xCBu ? 256u + b1 : op), op, b1, b2);
 }
 
+// ---------------------------------------------------------------------------
+// Fused records.  An instruction that only computes registers (no bus access,
+// no SP operand, no control flow but a jump whose target is known) is "pure".
+// A fused record holds up to kPure pure instructions that run one after the
+// other from pc, and the full record of the instruction after them, of any
+// kind: the step kernel takes them in one pass of its loop.  A pure
+// instruction needs eight words (gbx_exec.h exec_pure):
+//
+// p0  byte-permute selector of {W1:W0}: ALU operands x, y (bytes 0-1), 16-bit
+//     adder operand A (bytes 2-3)
+// p1  selector of the adder's operand B (bytes 0-1; bytes 2-3 read zero)
+// p2  [0:15] K, added in to y and to B (zero unless one of them is K)
+//     [16:31] of the first: main pc - pc; of the second: [16:23] cycles of
+//     the pure instructions, [24:31] their number
+// p3 p4 p5 p6 p7  the record's SW0, SW1, FL, CIW, SHW
+// ---------------------------------------------------------------------------
+constexpr uint32_t kPure = 2;
+constexpr int kPureWords = 8;
+constexpr int kFusedWords = kPure * kPureWords + kRecWords;
+struct Fused {
+  uint32_t w[kFusedWords];  // pure instructions, then the main record
+};
+__host__ __device__ constexpr bool pure_op(uint32_t op, uint32_t b1) {
+  const uint32_t z = op & 7u, y = (op >> 3) & 7u, p = op >> 4;
+  if (op == 0xCBu) return (b1 & 7u) != 6u;
+  if (op >= 0x40u && op < 0x80u) return y != 6u && z != 6u;  // LD r,r'
+  if (op >= 0x80u && op < 0xC0u) return z != 6u;             // ALU A,r
+  if (op >= 0xC0u) return z == 6u || op == 0xC3u || op == 0xF9u;  // ALU A,d8, JP a16, LD SP,HL
+  if (z == 4u || z == 5u || z == 6u) return y != 6u;         // INC r, DEC r, LD r,d8
+  if ((op & 0xFu) == 1u) return true;                        // LD rr,d16
+  if ((op & 0xFu) == 3u || (op & 0xFu) == 9u || (op & 0xFu) == 0xBu) return p != 3u;  // INC/DEC rr, ADD HL,rr
+  return op == 0x00u || op == 0x18u || op == 0x07u || op == 0x0Fu || op == 0x17u || op == 0x1Fu || op == 0x2Fu ||
+         op == 0x37u || op == 0x3Fu;
+}
+// The words of a pure instruction from its record (a jump's are NOP's).
+__host__ __device__ constexpr void pure_words(const Rec& r, uint32_t* p) {
+  const uint32_t yk = (r.w[4] >> 8) & 0xFFu, bk = (r.w[6] >> 16) & 0xFFu;
+  p[0] = (r.w[3] & 0xFFFFu) | (r.w[5] << 16);
+  p[1] = (r.w[5] >> 16) | (kZero4 << 16);
+  p[2] = (yk == Q_KL || bk == Q_KL) ? r.w[7] >> 16 : 0u;
+  p[3] = r.w[8];
+  p[4] = r.w[9];
+  p[5] = r.w[10];
+  p[6] = r.w[13];
+  p[7] = r.w[14];
+}
+// Start and extent of the pure instructions at offset i of an image.
+struct FusedRun {
+  uint32_t n = 0, cycles = 0, main = 0;
+  uint32_t at[kPure] = {};
+};
+// `end` bounds the offsets (from the window's start `lo`) at which a record
+// may be served; every instruction of the run and the one after it lies in
+// [lo, end).  A jump into the first 256 bytes of a window ends the run, since
+// the boot image may be mapped there.  JP a16 is followed with `abs_ok`: its
+// target as an offset of the image, which only a cart without bank switching
+// fixes (offsets below 0x8000 are then addresses).
+__host__ __device__ constexpr FusedRun fused_run(const uint8_t* img, uint32_t i, uint32_t lo, uint32_t end, bool abs_ok) {
+  FusedRun f{};
+  uint32_t pos = i;
+  while (f.n < kPure) {
+    const uint32_t op = img[pos], b1 = img[pos + 1], b2 = img[pos + 2];
+    if (!pure_op(op, b1)) break;
+    const Dec d = op == 0xCBu ? decode_cb(b1) : decode_op(op);
+    uint32_t next = pos + d.len;
+    if (op == 0x18u) {
+      next += sext8(b1);
+      if (next < lo + 0x100u || next >= lo + 0x4000u) break;
+    } else if (op == 0xC3u) {
+      next = b1 | (b2 << 8);
+      if (!abs_ok || (next & 0x3FFFu) < 0x100u || next >= 0x8000u || (next & 0x3FFFu) > 0x3FFDu) break;
+      lo = next & 0x4000u;
+      end = lo + 0x3FFEu;
+    }
+    if (next >= end) break;
+    f.at[f.n] = pos;
+    f.cycles += d.cyc;
+    ++f.n;
+    pos = next;
+  }
+  f.main = pos;
+  return f;
+}
+
 }  // namespace gbx

@@ -141,4 +141,31 @@ __device__ __forceinline__ ExecOut exec_insn(const Rec& r, const ExecIn& in) {
   return o;
 }
 
+// One pure instruction (gbx_decode.h) from its eight words: exec_insn's
+// operands, adders, logic, shifter, flags and writeback without the bus, the
+// stack, control flow and DAA.  sp keeps garbage above bit 15.
+__device__ __forceinline__ void exec_pure(const uint32_t* p, uint32_t& w0, uint32_t& w1, uint32_t& sp) {
+  const uint32_t W0 = w0, W1 = w1, K = p[2], FL = p[5], CIW = p[6], SHW = p[7];
+  const uint32_t XYA = perm(W1, W0, p[0]);
+  const uint32_t B16 = perm(W1, W0, p[1]) | K;
+  const uint32_t x = XYA & 0xFFu, A16 = XYA >> 16;
+  const uint32_t ym = ubfe((XYA | (K << 8)) ^ CIW, 8, 8);
+  const uint32_t s9 = x + ym + ubfe(W1 ^ CIW, CIW & 31u, 1);
+  const uint32_t rl = ((x | ym) & bit_mask<5>(CIW)) ^ (x & ym & bit_mask<6>(CIW));
+  const uint32_t XW = x | (x << 8);
+  const uint32_t rs = ubfe(perm(W1 << 19, XW, SHW), (SHW >> 16) & 31u, 8);
+  const uint32_t res = (s9 & (SHW >> 24)) | rs | rl;
+  // (K's upper half, the run's extent, only reaches bits 16-31 of the sum,
+  // which the carry vector takes out again and the writeback does not read)
+  const uint32_t sum = A16 + B16;
+  const uint32_t fsv = (s9 ^ x ^ ym) | perm(sum ^ A16 ^ B16, XW, CIW >> 16);
+  const uint32_t fw = (res == 0u ? 0x80u : 0u) | (ubfe(fsv, 4, 1) << 5) | (ubfe(fsv, 8, 1) << 4);
+  const uint32_t fn = (((fw & FL) | ((W1 >> 8) & ~FL)) & ubfe(FL, 8, 8)) ^ ubfe(FL, 16, 8);
+  const uint32_t U = (sum << 16) | (fn << 8) | res;
+  w0 = perm(U, W0, p[3]);
+  w1 = perm(U, W1, p[4]);
+  const uint32_t mspw = bit_mask<29>(FL);
+  sp = (sum & mspw) | (sp & ~mspw);
+}
+
 }  // namespace gbx

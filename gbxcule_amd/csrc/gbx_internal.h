@@ -90,6 +90,7 @@ struct DevState {
   const uint8_t* rom;       // ROM image, the 256-byte boot image, 16 KiB of 0xFF (open bus)
   const uint8_t* boot;
   const uint4* recs;        // pre-decoded instruction record per byte of the ROM buffer
+  const uint4* fused;       // fused record (pure instructions and the one after them) per byte
   int n, npad, obs_dim;
   int rom_banks, rom_mask, ram_banks, ram_bytes, cram_stride, mbc_kind;
   int step_lanes;       // envs per step-kernel wavefront: 64, 32, 16 or 8
@@ -102,6 +103,9 @@ struct StepArgs {
   int dbg_rst38, dbg_trap_pc, dbg_max_instr, dbg_watch;
 };
 
+// Fills s.recs and s.fused from the ROM buffer (`total` bytes: the ROM, the
+// boot image, the open-bus window).
+hipError_t launch_build_records(const DevState& s, int64_t total, hipStream_t st);
 hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st);
 hipError_t launch_render(const DevState& s, uint8_t* out, int64_t base, int packed,
                          hipStream_t st);

@@ -10,9 +10,17 @@
 // The implementation is not a translation of that kernel.  A wavefront runs
 // up to 64 independent instruction streams, so the loop body is built to
 // cost the same whatever mix of opcodes its lanes execute:
-//  * fetch + decode is four 16-byte loads of the pre-decoded 64-byte record
-//    of the instruction at pc (gbx_decode.h), issued for the next pc while
-//    the current instruction's writes, timer and PPU work run;
+//  * fetch + decode is eight 16-byte loads of the pre-decoded 128-byte fused
+//    record at pc (gbx_decode.h), issued for the next pc while the current
+//    instruction's writes, timer and PPU work run.  One pass of the loop runs
+//    the record's up to two register-only instructions and the instruction
+//    after them: bus address, read latency, write phase and timer are paid
+//    once for all (2.2-2.4 instructions a pass on the random-code carts, for
+//    about 100 more VALU instructions; 16,384 envs, frameskip 24: 128.0 ->
+//    102.9 ms; 64 envs, frameskip 4: 29.7 -> 20.1 ms).  Two, since a third
+//    finds a register-only instruction in few passes only, and two fill one
+//    128-byte line.  A pass whose register-only instructions would reach an
+//    event (event_budget) runs the instruction at pc alone;
 //  * execute is one straight-line datapath (gbx_exec.h) whose operands are
 //    byte permutes of the register file and the bus bytes selected by the
 //    record, with one shared adder, logic unit, shifter and 16-bit adder, so
@@ -60,6 +68,59 @@ constexpr DecTable make_dec_table() {
   return t;
 }
 __constant__ DecTable kDec = make_dec_table();
+
+// ---------------------------------------------------------------------------
+// Pre-decoded instruction records for the fetch: one 512-bit record and one
+// fused record (gbx_decode.h) per byte of the ROM buffer, from that byte and
+// the bytes after it in the same image (the ROM, the boot image, the open-bus
+// window).  Bytes past the end of an image read as 0; the kernel only uses a
+// record when all three instruction bytes lie inside one 16 KiB ROM window or
+// inside the boot image.
+// ---------------------------------------------------------------------------
+__device__ Rec record_at(const uint8_t* img, uint32_t len, uint32_t i, bool rom) {
+  const uint32_t op = img[i], b1 = i + 1u < len ? img[i + 1u] : 0u, b2 = i + 2u < len ? img[i + 2u] : 0u;
+  Rec r = bind_bytes(kDec.e[op == 0xCBu ? 256u + b1 : op], op, b1, b2);
+  // LY poll loops and block-copy loops whose bytes lie inside one 16 KiB window
+  if (rom && i + 5u < len) {
+    const uint32_t pl = poll_loop_len(img + i, min(8u, len - i));
+    if (pl != 0u && (i & 0x3FFFu) + pl <= 0x4000u) r = mark_poll_loop(r, img + i);
+    if ((i & 0x3FFFu) <= 0x3FF8u && i + 7u < len && copy_loop_at(img + i)) r = mark_copy_loop(r);
+  }
+  return r;
+}
+__global__ void build_records_kernel(const uint8_t* buf, uint32_t rom_bytes, uint32_t total, int abs_ok, uint4* recs,
+                                     uint4* fused) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= total) return;
+  const bool rom = i < rom_bytes, boot = !rom && i < rom_bytes + 0x100u;
+  const uint32_t base = rom ? 0u : boot ? rom_bytes : rom_bytes + 0x100u;
+  const uint32_t len = rom ? rom_bytes : boot ? 0x100u : total - base;
+  const uint8_t* img = buf + base;
+  const uint32_t k = i - base;
+  const uint32_t lo = rom ? k & ~0x3FFFu : 0u, end = lo + (boot ? 0xFEu : 0x3FFEu);
+  Fused f{};
+  FusedRun run{};
+  run.main = k;
+  if (k < end) run = fused_run(img, k, lo, end, rom && abs_ok != 0);
+  const Rec nop = kDec.e[0];
+  for (uint32_t j = 0; j < kPure; ++j) {
+    Rec r = nop;
+    if (j < run.n) {
+      r = record_at(img, len, run.at[j], rom);
+      if ((r.w[0] & 0xFFu) == 0x18u || (r.w[0] & 0xFFu) == 0xC3u) r = nop;
+    }
+    pure_words(r, f.w + j * kPureWords);
+  }
+  f.w[2] |= (run.main - k) << 16;
+  f.w[kPureWords + 2] |= (run.cycles | (run.n << 8)) << 16;
+  const Rec m = record_at(img, len, run.main, rom);
+  for (int j = 0; j < kRecWords; ++j) f.w[kPure * kPureWords + j] = m.w[j];
+  for (uint32_t j = 0; j < (uint32_t)kFusedWords / 4u; ++j)
+    fused[(size_t)i * (kFusedWords / 4) + j] = make_uint4(f.w[4 * j], f.w[4 * j + 1], f.w[4 * j + 2], f.w[4 * j + 3]);
+  const Rec own = record_at(img, len, k, rom);
+  for (uint32_t j = 0; j < (uint32_t)kRecWords / 4u; ++j)
+    recs[(size_t)i * (kRecWords / 4) + j] = make_uint4(own.w[4 * j], own.w[4 * j + 1], own.w[4 * j + 2], own.w[4 * j + 3]);
+}
 
 // ---------------------------------------------------------------------------
 // Buffer-resource access for the fixed-address state of a 64-env block: a
@@ -690,11 +751,14 @@ struct Lane {
     return const_cast<uint8_t*>(c ? cart_p + ((x - 0xA000u) << kEnvBlockShift)
                                   : memb + ((x << kEnvBlockShift) | lane));
   }
-  __device__ void write_bus(uint32_t n, uint32_t a0, uint32_t v0, uint32_t a1, uint32_t v1, bool& rv) {
+  // `before` runs ahead of a write with side effects.
+  template <typename F>
+  __device__ void write_bus(uint32_t n, uint32_t a0, uint32_t v0, uint32_t a1, uint32_t v1, bool& rv, F before) {
     const uint32_t x0 = a0 & 0xFFFFu, x1 = a1 & 0xFFFFu;
     const bool two = n >= 2u;
     const bool c0 = cart_plain(x0), c1 = cart_plain(x1);
     if (__builtin_expect((!(plain_store(x0) | c0)) | (two & !(plain_ram(x1) | c1)), 0)) {
+      before();
       write8(a0, v0);
       if (two) write8(a1, v1);
       if (mbc != MBC_ROM_ONLY) {
@@ -1146,7 +1210,7 @@ struct Lane {
 // spill VGPRs to scratch in the loop, and 131,072 envs in 64-lane
 // wavefronts are two per SIMD.
 template <int kMbc, bool kDbg, bool kCram = true>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MBC_ROM_ONLY && kCram) ? 2 : 3))) void step_kernel(DevState s, StepArgs args) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void step_kernel(DevState s, StepArgs args) {
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (uint32_t)s.n) return;
   Lane L{s};
@@ -1166,7 +1230,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
   L.rcs = make_rsrc(s.cs + (size_t)blk * (kCartStateStride * kEnvBlock),
                     kCartStateStride * kEnvBlock * 4);
   const rsrc_t rcnt = make_rsrc(s.cnt + (size_t)blk * (2 * kEnvBlock), 2 * kEnvBlock * 8);
-  const uint4* recs = in_vgpr(reinterpret_cast<const uint4*>(s.recs));  // 4 per record
+  const uint4* recs = in_vgpr(reinterpret_cast<const uint4*>(s.recs));    // 4 per record
+  const uint4* fused = in_vgpr(reinterpret_cast<const uint4*>(s.fused));  // 8 per fused record
 
   // ---- load (cpu_step_builder.py:930-967) ---------------------------------
   L.pc = (uint32_t)L.SC(F_PC) & 0xFFFFu;
@@ -1248,18 +1313,43 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
   const int frames = (int)in_vgpr((uint32_t)args.frames);
   constexpr bool dbg = kDbg;
 
-  // record of the instruction at pc (valid when rv)
+  // record of the instruction at pc, with the pure instructions that run
+  // before it (valid when rv; the debug variants run every instruction alone)
   Rec rec{};
+  uint32_t pure[kPure * kPureWords];
   bool rv = false;
-  auto load_rec = [&](uint32_t i) {
-    const uint4* p = recs + (size_t)i * 4u;
+  auto ld_words = [&](const uint4* p, uint32_t* w, int quads) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
+    for (int k = 0; k < quads; ++k) {
       const u32x4 q = ld_global(reinterpret_cast<const u32x4*>(p + k));
-      rec.w[4 * k] = q[0];
-      rec.w[4 * k + 1] = q[1];
-      rec.w[4 * k + 2] = q[2];
-      rec.w[4 * k + 3] = q[3];
+      w[4 * k] = q[0];
+      w[4 * k + 1] = q[1];
+      w[4 * k + 2] = q[2];
+      w[4 * k + 3] = q[3];
+    }
+  };
+  auto load_single = [&](uint32_t i) { ld_words(recs + (size_t)i * (kRecWords / 4), rec.w, kRecWords / 4); };
+  auto load_rec = [&](uint32_t i) {
+    if (kDbg) {
+      load_single(i);
+    } else {
+      const uint4* p = fused + (size_t)i * (kFusedWords / 4);
+      ld_words(p, pure, kPure * kPureWords / 4);
+      ld_words(p + kPure * kPureWords / 4, rec.w, kRecWords / 4);
+    }
+  };
+  // no pure instruction ahead of the record
+  auto clear_pure = [&]() {
+#pragma unroll
+    for (uint32_t j = 0; j < kPure; ++j) {
+      uint32_t* p = pure + j * kPureWords;
+      p[0] = p[1] = kZero4;
+      p[2] = 0u;
+      p[3] = 0x03020100u;
+      p[4] = 0x03020000u | (U_FN << 8);
+      p[5] = FALL << 8;
+      p[6] = 9u | 0x0C0C0000u;
+      p[7] = 0x0C0Cu;
     }
   };
 
@@ -1316,21 +1406,46 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
     // write the RTC registers (the reference ticks it after every step)
     int rtc_pre = 0;
     uint32_t op = 0;
-    const uint32_t pc_before = L.pc;
+    uint32_t pc_before = L.pc;
+    // cycles of the pure instructions run this pass and not yet counted; the
+    // budget covers them, so counting them is what the fast tail does
+    uint32_t cp = 0;
+    auto count_pure = [&]() {
+      L.div = (L.div + cp) & 0xFFFFu;
+      L.scan += (L.lcdc & 0x80u) ? cp : 0u;
+      if (kMbc == MBC_MBC3) L.rtc_sub += L.rtc_halt ? 0 : (int)cp;
+      ncyc += cp;
+      cframe += (int)cp;
+      L.budget -= (int)cp;
+      cp = 0;
+    };
     // pending bus writes: the instruction's, then the interrupt push
     uint32_t wn = 0, wa0 = 0, wv0 = 0, wa1 = 0, wv1 = 0;
 
     if (__builtin_expect(!hiter, 1)) {
       // ---- fetch + decode ------------------------------------------------------
-      const uint32_t pc = L.pc;
+      uint32_t pc = L.pc;
       // (rare branches of the per-instruction path test a wave-uniform
       // ballot first: when no lane takes them the path keeps its exec mask
       // instead of saving and restoring it around a skipped block)
-      if (__builtin_expect(__ballot(!rv) != 0u, 0)) {
-        if (!rv) {
-          if (L.rec_ok(pc)) load_rec(L.rec_index(pc));
+      if (!kDbg) cp = ubfe(pure[kPureWords + 2], 16, 8);
+      // no valid record, or an event within the pure instructions: the
+      // instruction at pc alone
+      const bool single = !rv | ((!kDbg) & (cp != 0u) & ((int)cp >= L.budget));
+      if (__builtin_expect(__ballot(single) != 0u, 0)) {
+        if (single) {
+          if (L.rec_ok(pc)) load_single(L.rec_index(pc));
           else rec = L.fetch_slow();
+          if (!kDbg) clear_pure();
+          cp = 0;
         }
+      }
+      if (!kDbg) {
+        exec_pure(pure, L.w0, L.w1, L.sp);
+        exec_pure(pure + kPureWords, L.w0, L.w1, L.sp);
+        pc = (pc + (pure[2] >> 16)) & 0xFFFFu;
+        pc_before = pc;
+        ninstr += pure[kPureWords + 2] >> 24;
       }
       op = rec.w[0] & 0xFFu;
       if (dbg) {  // debug traps before execution: the instruction does not run
@@ -1375,6 +1490,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
         const bool h1 = (nr > 1u) & ((x1 & 0xFFBAu) == 0xFF00u) & (x1 > 0xFF01u);
         uint32_t r0 = v0, r1 = v1;
         if (__builtin_expect(__ballot(h0 | h1) != 0u, 0)) {
+          if (h0 | h1) count_pure();
           r0 = h0 ? L.read_ppu(x0, v0) : v0;
           r1 = h1 ? L.read_ppu(x1, v1) : v1;
         }
@@ -1398,6 +1514,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
       // that is executing an instruction)
       if (__builtin_expect(__ballot(o.misc != 0u) != 0u, 0)) {
         if (o.misc != 0u) {  // DI EI RETI HALT, illegal opcodes, poll/copy loops
+          count_pure();
           L.settle();  // the fast-forwards start from the PPU and timer state
           if (o.misc & 1u) {
             L.ime = (o.misc >> 1) & 1u;
@@ -1485,7 +1602,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
 
     // ---- write phase, debug checks, timer, PPU, interrupt check --------------
     int svc = 0;
-    if (__builtin_expect(wn != 0u, 1)) L.write_bus(wn, wa0, wv0, wa1, wv1, rv);
+    if (__builtin_expect(wn != 0u, 1)) L.write_bus(wn, wa0, wv0, wa1, wv1, rv, count_pure);
     if (dbg) {
       if (!hiter) {
         if (dbg_rst38 && L.pc >= 0xFE00u && !trap) {
@@ -1510,20 +1627,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
     // to the nearest of those events, and 0 while any of them is pending or
     // once this step made one (an IO, MBC or RTC write, a trap).
     const uint32_t lc_now = L.lcdc;
-    const uint32_t ucyc = (uint32_t)cycles;
+    const uint32_t ucyc = (uint32_t)cycles + cp;
     const bool lcd_on = (lc_now & 0x80u) != 0u;
-    const bool fast = (trap == 0) & (cycles < L.budget);
+    const bool fast = (trap == 0) & ((int)ucyc < L.budget);
     if (__builtin_expect(fast, 1)) {
       // stat_fresh, lyc_pp and lcd_pp already hold what a PPU step would set:
       // STAT, LYC and LCDC writes go through io_write, which zeroes the
       // budget, and a launch starts with the budget at 0
       L.div = (L.div + ucyc) & 0xFFFFu;
       L.scan = lcd_on ? L.scan + ucyc : 0u;
-      if (kMbc == MBC_MBC3) L.rtc_sub += L.rtc_halt ? 0 : cycles;
+      if (kMbc == MBC_MBC3) L.rtc_sub += L.rtc_halt ? 0 : (int)ucyc;
       ncyc += ucyc;
-      cframe += cycles;
-      L.budget -= cycles;
+      cframe += (int)ucyc;
+      L.budget -= (int)ucyc;
     } else if (!trap) {
+      count_pure();
       L.settle();
       L.timer_tick(cycles);
       if (!hiter & (L.ime_delay != 0u)) {
@@ -1687,6 +1805,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((kMbc != MB
 }
 
 }  // namespace
+
+hipError_t launch_build_records(const DevState& s, int64_t total, hipStream_t st) {
+  hipLaunchKernelGGL(build_records_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, s.rom,
+                     (uint32_t)s.rom_len, (uint32_t)total, s.mbc_kind == MBC_ROM_ONLY ? 1 : 0,
+                     const_cast<uint4*>(s.recs), const_cast<uint4*>(s.fused));
+  return hipGetLastError();
+}
 
 hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st) {
   if (s.n <= 0) return hipSuccess;

@@ -74,6 +74,30 @@ void harness_exec(const uint32_t* in, uint32_t* out) {
   for (int k = 0; k < 12; ++k) out[k] = res[k];
 }
 
+// out: [is pure, its eight words]
+void harness_pure_words(uint32_t op, uint32_t b1, uint32_t b2, uint32_t* out) {
+  out[0] = gbx::pure_op(op, b1) ? 1u : 0u;
+  gbx::pure_words(gbx::decode_insn(op, b1, b2), out + 1);
+}
+
+// in: pure words[8], w0, w1, sp (11 words); out: w0, w1, sp
+void harness_pure(const uint32_t* in, uint32_t* out) {
+  uint32_t w0 = in[8], w1 = in[9], sp = in[10];
+  gbx::exec_pure(in, w0, w1, sp);
+  out[0] = w0;
+  out[1] = w1;
+  out[2] = sp & 0xFFFFu;
+}
+
+// out: [number of pure instructions, cycles, main offset, their offsets]
+void harness_fused(const uint8_t* img, uint32_t i, uint32_t lo, uint32_t end, uint32_t abs_ok, uint32_t* out) {
+  const gbx::FusedRun f = gbx::fused_run(img, i, lo, end, abs_ok != 0);
+  out[0] = f.n;
+  out[1] = f.cycles;
+  out[2] = f.main;
+  for (uint32_t j = 0; j < gbx::kPure; ++j) out[3 + j] = f.at[j];
+}
+
 // out: [poll-loop length in bytes (0: none), FL word, DW word] of the decoded and marked
 // record at p (n bytes readable)
 void harness_poll(const uint8_t* p, uint32_t n, uint32_t* out) {

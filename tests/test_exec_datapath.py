@@ -46,6 +46,9 @@ def harness(tmp_path_factory):
     lib.harness_exec.argtypes = [u32p, u32p]
     lib.harness_poll.argtypes = [ctypes.c_char_p, ctypes.c_uint32, u32p]
     lib.harness_copy.argtypes = [ctypes.c_char_p, u32p]
+    lib.harness_pure_words.argtypes = [ctypes.c_uint32] * 3 + [u32p]
+    lib.harness_pure.argtypes = [u32p, u32p]
+    lib.harness_fused.argtypes = [ctypes.c_char_p] + [ctypes.c_uint32] * 4 + [u32p]
     return lib
 
 
@@ -303,3 +306,78 @@ def test_copy_loops_in_carts_are_marked(harness):
     assert marked(cart_c3(2)) == 4
     for case in CASES:
         assert marked(copy_cart(*case)) == (13 if case[5] else 12)
+
+
+@pytest.mark.parametrize("seed", [21, 22])
+def test_pure_datapath_matches_datapath(harness, seed):
+    """Every pure instruction, from random registers and immediates, through
+    exec_pure and through exec_insn: the same registers and SP, no bus access,
+    no effect beyond them.  The run's extent in p2's upper half must not show."""
+    rng = np.random.default_rng(seed)
+    rec, words, res, out, pout = _arr(16), _arr(9), _arr(12), _arr(12), _arr(3)
+    pures = 0
+    for op in OPS:
+        for _ in range(24):
+            b = [int(x) for x in rng.integers(0, 256, 2)]
+            if op & 0x100:
+                code = [0xCB, op & 0xFF, b[1]]
+            else:
+                code = [op, *b]
+            harness.harness_pure_words(*code, words)
+            if not words[0]:
+                break
+            harness.harness_decode(*code, rec)
+            w = [int(x) for x in rng.integers(0, 2**32, 2)]
+            w[1] &= 0xFFFFF0FF  # F's low bits are zero
+            sp, pc = (int(x) for x in rng.integers(0, 0x10000, 2))
+            rin = (ctypes.c_uint32 * 22)(*rec, *w, sp, pc, 0x5A, 0xA5)
+            harness.harness_exec(rin, res)
+            assert (rec[7] >> 8) & 3 == 0 and res[6] == 0 and res[11] == 0, code  # no reads, writes, IME/HALT/trap
+            meta = int(rng.integers(0, 0x10000)) << 16
+            pw = list(words)[1:]
+            jump = op in (0x18, 0xC3)
+            if not jump:
+                assert res[4] == (pc + (rec[0] >> 24 & 3)) & 0xFFFF, code
+                pw[2] |= meta
+                harness.harness_pure((ctypes.c_uint32 * 11)(*pw, *w, sp), pout)
+                assert (pout[0], pout[1], pout[2]) == (res[1], res[2], res[3]), code
+            else:
+                assert (res[1], res[2], res[3]) == (w[0], w[1], sp), code
+        pures += int(words[0])
+    # CB on a register 224; LD r,r' 49; ALU A,r 56 and A,d8 8; INC/DEC r 14; LD
+    # r,d8 7; LD rr,d16 4; INC/DEC rr 6; ADD HL,rr 3; rotates of A 4; CPL SCF
+    # CCF 3; NOP, JR, JP a16, LD SP,HL
+    assert pures == 382
+
+
+def test_fused_runs(harness):
+    """Runs end at an instruction that is not pure, at the window's end, at a
+    jump out of the window or into its first 256 bytes, after two."""
+    out = _arr(5)
+
+    def run(code, at=0x200, lo=0, end=0x3FFE, abs_ok=1, size=0x8000):
+        img = bytearray([0x76]) * size
+        for a, c in code.items():
+            img[a : a + len(c)] = c
+        harness.harness_fused(bytes(img), at, lo, end, abs_ok, out)
+        return tuple(out)[: 3 + out[0]]
+
+    assert run({0x200: b"\x76"}) == (0, 0, 0x200)
+    assert run({0x200: b"\x78\x34"}) == (1, 4, 0x201, 0x200)
+    assert run({0x200: b"\x78\x01\x34\x12\x04"}) == (2, 16, 0x204, 0x200, 0x201)
+    assert run({0x200: b"\xcb\x37\xcb\x36"}) == (1, 8, 0x202, 0x200)
+    # the instruction after the run must have a record too
+    assert run({0x3FFC: b"\x78\x78\x78"}, at=0x3FFC) == (1, 4, 0x3FFD, 0x3FFC)
+    assert run({0x3FFD: b"\x3e\x00"}, at=0x3FFD) == (0, 0, 0x3FFD)
+    # JR inside the window, out of it, into its first 256 bytes
+    assert run({0x200: b"\x18\x10", 0x212: b"\x04"}) == (2, 16, 0x213, 0x200, 0x212)
+    assert run({0x4110: b"\x18\x80"}, at=0x4110, lo=0x4000, end=0x7FFE) == (0, 0, 0x4110)
+    assert run({0x3FF0: b"\x18\x20"}, at=0x3FF0) == (0, 0, 0x3FF0)
+    # JP: followed only where offsets are addresses; into the other window and
+    # to its end; not above the ROM, nor below 0x100
+    assert run({0x200: b"\xc3\x00\x03"}) == (1, 16, 0x300, 0x200)
+    assert run({0x200: b"\xc3\x00\x03"}, abs_ok=0) == (0, 0, 0x200)
+    assert run({0x200: b"\xc3\xfc\x7f", 0x7FFC: b"\x78\x78"}) == (2, 20, 0x7FFD, 0x200, 0x7FFC)
+    assert run({0x200: b"\xc3\xfe\x7f"}) == (0, 0, 0x200)
+    assert run({0x200: b"\xc3\x00\xc0"}) == (0, 0, 0x200)
+    assert run({0x200: b"\xc3\x50\x00"}) == (0, 0, 0x200)

@@ -148,9 +148,21 @@ hipError_t dalloc(T** p, size_t count) {
   return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T) > 0 ? count * sizeof(T) : 1);
 }
 
-// The ROM buffer is the ROM, then the boot image, then one 16 KiB window of
-// 0xFF that an unmapped ROM bank reads (open bus).
-constexpr int64_t kOpenBusBytes = 0x4000;
+// The ROM buffer, in 16 KiB windows: the ROM, one of 0xFF that an unmapped
+// ROM bank reads (open bus), and the banks that the window at 0000 can hold
+// (bank 0, and on an MBC1 cart banks 32, 64 and 96) with the boot image over
+// their first 256 bytes.
+std::vector<uint8_t> rom_buffer(const uint8_t* rom, int64_t rom_bytes, const uint8_t* boot, int kind) {
+  std::vector<uint8_t> b(rom, rom + rom_bytes);
+  b.resize(b.size() + 0x4000, 0xFF);
+  const int64_t views = kind == MBC_MBC1 ? std::min<int64_t>(4, std::max<int64_t>(1, rom_bytes >> 19)) : 1;
+  for (int64_t k = 0; k < views; ++k) {
+    const uint8_t* bank = rom + (k << 19);
+    b.insert(b.end(), boot, boot + 0x100);
+    b.insert(b.end(), bank + 0x100, bank + 0x4000);
+  }
+  return b;
+}
 
 // Header parse (reference core/cartridge.py:139-187).
 int parse_header(const uint8_t* rom, int64_t rom_len, int* kind, int64_t* rom_bytes,
@@ -259,10 +271,12 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   uint8_t *drom = nullptr, *dboot = nullptr;
   Rec* drecs = nullptr;
   Fused* dfused = nullptr;
-  A(dalloc(&drom, (size_t)(rom_bytes + 0x100 + kOpenBusBytes)));
+  const std::vector<uint8_t> rombuf = rom_buffer(rom, rom_bytes, boot, kind);
+  s.no_rec = (int64_t)rombuf.size();
+  A(dalloc(&drom, rombuf.size()));
   A(dalloc(&dboot, (size_t)0x100));
-  A(dalloc(&drecs, (size_t)(rom_bytes + 0x100 + kOpenBusBytes)));
-  A(dalloc(&dfused, (size_t)(rom_bytes + 0x100 + kOpenBusBytes)));
+  A(dalloc(&drecs, rombuf.size()));
+  A(dalloc(&dfused, rombuf.size() + 1));
   s.rom = drom;
   s.boot = dboot;
   s.recs = reinterpret_cast<const uint4*>(drecs);
@@ -280,11 +294,9 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
     free_ctx(c);
     return fail(GBX_E_HIP, std::string("device allocation failed: ") + hipGetErrorString(e));
   }
-  A(hipMemcpy(drom, rom, (size_t)rom_bytes, hipMemcpyHostToDevice));
-  A(hipMemcpy(drom + rom_bytes, boot, 0x100, hipMemcpyHostToDevice));
-  A(hipMemset(drom + rom_bytes + 0x100, 0xFF, (size_t)kOpenBusBytes));
+  A(hipMemcpy(drom, rombuf.data(), rombuf.size(), hipMemcpyHostToDevice));
   A(hipMemcpy(dboot, boot, 0x100, hipMemcpyHostToDevice));
-  A(launch_build_records(s, rom_bytes + 0x100 + kOpenBusBytes, nullptr));
+  A(launch_build_records(s, nullptr));
   const HashHost& hh = hash_host();
   A(hipMemcpy(c->hash.digits, hh.digits.data(), hh.digits.size(), hipMemcpyHostToDevice));
   A(hipMemcpy(c->hash.fields, hh.fields.data(), hh.fields.size() * 8, hipMemcpyHostToDevice));

@@ -76,6 +76,11 @@ constexpr uint32_t kZero4 = 0x0C0C0C0Cu;
 // flag bits of F
 constexpr uint32_t FZ = 0x80, FN = 0x40, FH = 0x20, FC = 0x10, FALL = 0xF0;
 
+// FL bits of the effects outside the datapath
+constexpr uint32_t kMiscIme = 1u << 24, kMiscImeOn = 1u << 25, kMiscHalt = 1u << 26, kMiscTrap = 1u << 27,
+                   kMiscLoop = 1u << 28, kMiscDaa = 1u << 30;
+constexpr uint32_t kMisc = kMiscIme | kMiscImeOn | kMiscHalt | kMiscTrap | kMiscLoop | kMiscDaa;
+
 // How K is bound from the instruction bytes.
 enum KMode : uint32_t { KM_CONST = 0, KM_IMM8, KM_IMM16, KM_HIGH, KM_SEXT, KM_REL };
 // Branch condition (bit of W1 ^ TW that decides "taken").
@@ -336,7 +341,7 @@ __host__ __device__ constexpr Dec decode_op(uint32_t op) {
       set_shift(d, y); set_x(d, 7); set_dst(d, 7); d.E = FC; d.M = FC;
       return d;
     case 0x27:  // DAA (alu.py:897-950): N kept, H cleared, Z and C computed
-      set_x(d, 7); set_mov(d); set_dst(d, 7); d.daa = 1; d.E = FZ | FC; d.M = FZ | FN | FC;
+      d.daa = 1;
       return d;
     case 0x2F:  // CPL: x XOR 0xFF, N and H set
       set_x(d, 7); set_y(d, 8); d.k = 0xFF; d.lor = 1; d.land = 1; set_dst(d, 7);
@@ -472,7 +477,7 @@ __host__ __device__ constexpr uint32_t poll_loop_len(const uint8_t* p, uint32_t 
     return n + 5u;
   return 0;
 }
-constexpr uint32_t kPollFlag = 1u << 28;
+constexpr uint32_t kPollFlag = kMiscLoop;
 __host__ __device__ constexpr Rec mark_poll_loop(Rec r, const uint8_t* p) {
   const uint32_t n = p[0] == 0xF0u ? 2u : 3u;
   const uint32_t j = p[n + 2];
@@ -532,19 +537,32 @@ __host__ __device__ constexpr Rec decode_insn(uint32_t op, uint32_t b1, uint32_t
 // A fused record holds up to kPure pure instructions that run one after the
 // other from pc, and the full record of the instruction after them, of any
 // kind: the step kernel takes them in one pass of its loop.  A pure
-// instruction needs eight words (gbx_exec.h exec_pure):
+// instruction needs eight words (gbx_exec.h exec_pure).  Each packs operands
+// of several datapath instructions, at the bits where they use them:
 //
 // p0  byte-permute selector of {W1:W0}: ALU operands x, y (bytes 0-1), 16-bit
 //     adder operand A (bytes 2-3)
-// p1  selector of the adder's operand B (bytes 0-1; bytes 2-3 read zero)
-// p2  [0:15] K, added in to y and to B (zero unless one of them is K)
-//     [16:31] of the first: main pc - pc; of the second: [16:23] cycles of
-//     the pure instructions, [24:31] their number
-// p3 p4 p5 p6 p7  the record's SW0, SW1, FL, CIW, SHW
+// p1  [16:31] selector of the adder's operand B; [0:15] flag-source selector
+//     of x and y: H from bit 4 of byte 0, C from bit 0 of byte 1
+// p2  [0:4] carry-in bit of W1 ^ p6  [5] logic OR term  [6] logic AND term
+//     [7] SP takes the 16-bit sum  [8:15] immediate ORed into y  [16:31] K,
+//     ORed into B
+// p3  p4  writeback selectors of W0, W1
+// p5  [0:4] 16 + shift  [8:15] computed flags taken  [16:31] shifter selector
+// p6  [0:8] subtract mask (0x1FF: y complemented, bit 8 a borrow)
+//     [12] carry-in inverted
+// p7  [0:7] adder result mask  [8:15] flags kept  [16:31] of the first
+//     instruction: cycles of the pure instructions, their number << 8, or
+//     kNoRecord; of the second: main pc - pc
+//
+// ADD HL,rr and the SP forms are left out: they alone take flags from the
+// 16-bit adder, whose carries then need no instructions here.
 // ---------------------------------------------------------------------------
 constexpr uint32_t kPure = 2;
 constexpr int kPureWords = 8;
 constexpr int kFusedWords = kPure * kPureWords + kRecWords;
+// In p7 of the first: no record here (more cycles than any run has).
+constexpr uint32_t kNoRecord = 0xFFu << 16;
 struct Fused {
   uint32_t w[kFusedWords];  // pure instructions, then the main record
 };
@@ -556,21 +574,59 @@ __host__ __device__ constexpr bool pure_op(uint32_t op, uint32_t b1) {
   if (op >= 0xC0u) return z == 6u || op == 0xC3u || op == 0xF9u;  // ALU A,d8, JP a16, LD SP,HL
   if (z == 4u || z == 5u || z == 6u) return y != 6u;         // INC r, DEC r, LD r,d8
   if ((op & 0xFu) == 1u) return true;                        // LD rr,d16
-  if ((op & 0xFu) == 3u || (op & 0xFu) == 9u || (op & 0xFu) == 0xBu) return p != 3u;  // INC/DEC rr, ADD HL,rr
+  if ((op & 0xFu) == 3u || (op & 0xFu) == 0xBu) return p != 3u;  // INC/DEC rr
   return op == 0x00u || op == 0x18u || op == 0x07u || op == 0x0Fu || op == 0x17u || op == 0x1Fu || op == 0x2Fu ||
          op == 0x37u || op == 0x3Fu;
 }
-// The words of a pure instruction from its record (a jump's are NOP's).
-__host__ __device__ constexpr void pure_words(const Rec& r, uint32_t* p) {
-  const uint32_t yk = (r.w[4] >> 8) & 0xFFu, bk = (r.w[6] >> 16) & 0xFFu;
-  p[0] = (r.w[3] & 0xFFFFu) | (r.w[5] << 16);
-  p[1] = (r.w[5] >> 16) | (kZero4 << 16);
-  p[2] = (yk == Q_KL || bk == Q_KL) ? r.w[7] >> 16 : 0u;
-  p[3] = r.w[8];
-  p[4] = r.w[9];
-  p[5] = r.w[10];
-  p[6] = r.w[13];
-  p[7] = r.w[14];
+// The words of the pure instruction op, b1, b2 (a jump's are NOP's).
+__host__ __device__ constexpr void pure_words(uint32_t op, uint32_t b1, uint32_t b2, uint32_t* p) {
+  if (op == 0x18u || op == 0xC3u) op = 0u;
+  Dec d = op == 0xCBu ? decode_cb(b1) : decode_op(op);
+  const uint32_t k = d.kmode == KM_IMM8 ? b1 : d.kmode == KM_IMM16 ? b1 | (b2 << 8) : d.k;
+  uint32_t ky = ((d.xyq >> 8) & 0xFFu) == Q_KL ? k & 0xFFu : 0u;
+  const uint32_t kb = ((d.abq >> 16) & 0xFFu) == Q_KL ? k & 0xFFFFu : 0u;
+  // flags taken from the computed ones (N always computes as 1) and kept
+  uint32_t taken = d.E & d.M, kept = ~d.E & d.M & FALL;
+  uint32_t sub = d.subm ? 0x1FFu : 0u, cin = d.cipos == 12u ? 12u : 8u;
+  uint32_t xy = d.xyp & 0xFFFFu, fsel = d.fsel;
+  if (d.X & FN) taken |= FN;
+  if ((d.X & FH) && !(d.E & FH)) {  // AND, BIT, CPL: H set
+    taken |= FH;
+    fsel = set_byte(fsel, 0, SELFF);
+  }
+  if (d.sh != 0u) {  // shifts: y = x, and x - x leaves no carries
+    xy = (xy & 0xFFu) * 0x101u;
+    sub = 0x1FFu;
+  }
+  uint32_t inv = (cin == 12u && d.subm) ? 1u << 12 : 0u;  // SBC
+  if (op == 0x37u) {  // SCF
+    taken |= FC;
+    fsel = set_byte(fsel, 1, SELFF);
+  }
+  if (op == 0x3Fu) {  // CCF: 0 + FF + !C carries when C is clear
+    taken |= FC;
+    kept &= ~FC;
+    ky = 0xFFu;
+    cin = 12u;
+    inv = 1u << 12;
+  }
+  p[0] = xy | (d.abp << 16);
+  p[1] = (fsel & 0xFFFFu) | (d.abp & 0xFFFF0000u);
+  p[2] = cin | (d.lor << 5) | (d.land << 6) | (d.spw << 7) | (ky << 8) | (kb << 16);
+  p[3] = d.sw0;
+  p[4] = d.sw1;
+  p[5] = (16u + d.sh) | (taken << 8) | (d.shsel << 16);
+  p[6] = sub | inv;
+  p[7] = d.madd | (kept << 8);
+}
+// The words that leave everything as it is (NOP's).
+struct PureWords {
+  uint32_t w[kPureWords];
+};
+__host__ __device__ constexpr PureWords no_pure() {
+  PureWords p{};
+  pure_words(0u, 0u, 0u, p.w);
+  return p;
 }
 // Start and extent of the pure instructions at offset i of an image.
 struct FusedRun {

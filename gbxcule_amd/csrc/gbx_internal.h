@@ -87,7 +87,9 @@ struct DevState {
   uint8_t* pix_packed;  // [n][72][20]
   uint8_t* latches;     // [144][kLatchStride] env-0 scanline latches, one 16-byte entry per line
   uint8_t* frame_bg;    // [144][160] env-0 full-frame shades
-  const uint8_t* rom;       // ROM image, the 256-byte boot image, 16 KiB of 0xFF (open bus)
+  // 16 KiB windows: the ROM; one of 0xFF (open bus); copies of the banks that
+  // window 0 can hold, with the boot image in their first 256 bytes
+  const uint8_t* rom;
   const uint8_t* boot;
   const uint4* recs;        // pre-decoded instruction record per byte of the ROM buffer
   const uint4* fused;       // fused record (pure instructions and the one after them) per byte
@@ -95,6 +97,7 @@ struct DevState {
   int rom_banks, rom_mask, ram_banks, ram_bytes, cram_stride, mbc_kind;
   int step_lanes;       // envs per step-kernel wavefront: 64, 32, 16 or 8
   int64_t rom_len;
+  int64_t no_rec;       // bytes of the ROM buffer, the fused record that serves no pc
 };
 
 struct StepArgs {
@@ -103,9 +106,8 @@ struct StepArgs {
   int dbg_rst38, dbg_trap_pc, dbg_max_instr, dbg_watch;
 };
 
-// Fills s.recs and s.fused from the ROM buffer (`total` bytes: the ROM, the
-// boot image, the open-bus window).
-hipError_t launch_build_records(const DevState& s, int64_t total, hipStream_t st);
+// Fills s.recs and s.fused from the ROM buffer.
+hipError_t launch_build_records(const DevState& s, hipStream_t st);
 hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st);
 hipError_t launch_render(const DevState& s, uint8_t* out, int64_t base, int packed,
                          hipStream_t st);

@@ -16,11 +16,14 @@
 //    the record's up to two register-only instructions and the instruction
 //    after them: bus address, read latency, write phase and timer are paid
 //    once for all (2.2-2.4 instructions a pass on the random-code carts, for
-//    about 100 more VALU instructions; 16,384 envs, frameskip 24: 128.0 ->
-//    102.9 ms; 64 envs, frameskip 4: 29.7 -> 20.1 ms).  Two, since a third
-//    finds a register-only instruction in few passes only, and two fill one
-//    128-byte line.  A pass whose register-only instructions would reach an
-//    event (event_budget) runs the instruction at pc alone;
+//    about 75 more VALU instructions; 16,384 envs, frameskip 24: 128.0 -> 85.4
+//    ms; 64 envs, frameskip 4: 29.7 -> 17.4 ms).  Two, since a third finds a
+//    register-only instruction in few passes only, and two fill one 128-byte
+//    line.  A pass whose register-only instructions would reach an event
+//    (event_budget) runs the instruction at pc alone;
+//  * what an instruction computes without the bytes it reads (carry-in,
+//    branch, SP, write addresses) is pinned behind the issue of the read,
+//    whose latency covers it;
 //  * execute is one straight-line datapath (gbx_exec.h) whose operands are
 //    byte permutes of the register file and the bus bytes selected by the
 //    record, with one shared adder, logic unit, shifter and 16-bit adder, so
@@ -72,52 +75,52 @@ __constant__ DecTable kDec = make_dec_table();
 // ---------------------------------------------------------------------------
 // Pre-decoded instruction records for the fetch: one 512-bit record and one
 // fused record (gbx_decode.h) per byte of the ROM buffer, from that byte and
-// the bytes after it in the same image (the ROM, the boot image, the open-bus
-// window).  Bytes past the end of an image read as 0; the kernel only uses a
-// record when all three instruction bytes lie inside one 16 KiB ROM window or
-// inside the boot image.
+// the bytes after it in the same 16 KiB window.  Bytes past the end of a
+// window read as 0; the kernel only uses a record when all three instruction
+// bytes lie inside one window.  One more fused record serves no pc.
 // ---------------------------------------------------------------------------
-__device__ Rec record_at(const uint8_t* img, uint32_t len, uint32_t i, bool rom) {
-  const uint32_t op = img[i], b1 = i + 1u < len ? img[i + 1u] : 0u, b2 = i + 2u < len ? img[i + 2u] : 0u;
+__device__ Rec record_at(const uint8_t* img, uint32_t i, uint32_t loops_from) {
+  const uint32_t op = img[i], b1 = i + 1u < 0x4000u ? img[i + 1u] : 0u, b2 = i + 2u < 0x4000u ? img[i + 2u] : 0u;
   Rec r = bind_bytes(kDec.e[op == 0xCBu ? 256u + b1 : op], op, b1, b2);
-  // LY poll loops and block-copy loops whose bytes lie inside one 16 KiB window
-  if (rom && i + 5u < len) {
-    const uint32_t pl = poll_loop_len(img + i, min(8u, len - i));
-    if (pl != 0u && (i & 0x3FFFu) + pl <= 0x4000u) r = mark_poll_loop(r, img + i);
-    if ((i & 0x3FFFu) <= 0x3FF8u && i + 7u < len && copy_loop_at(img + i)) r = mark_copy_loop(r);
+  // LY poll loops and block-copy loops whose bytes lie inside the window
+  if (i >= loops_from && i + 5u < 0x4000u) {
+    if (poll_loop_len(img + i, min(8u, 0x4000u - i)) != 0u) r = mark_poll_loop(r, img + i);
+    if (i <= 0x3FF8u && copy_loop_at(img + i)) r = mark_copy_loop(r);
   }
   return r;
 }
-__global__ void build_records_kernel(const uint8_t* buf, uint32_t rom_bytes, uint32_t total, int abs_ok, uint4* recs,
+__global__ void build_records_kernel(const uint8_t* buf, uint32_t rom_bytes, uint32_t total, int rom_only, uint4* recs,
                                      uint4* fused) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  const bool rom = i < rom_bytes, boot = !rom && i < rom_bytes + 0x100u;
-  const uint32_t base = rom ? 0u : boot ? rom_bytes : rom_bytes + 0x100u;
-  const uint32_t len = rom ? rom_bytes : boot ? 0x100u : total - base;
-  const uint8_t* img = buf + base;
-  const uint32_t k = i - base;
-  const uint32_t lo = rom ? k & ~0x3FFFu : 0u, end = lo + (boot ? 0xFEu : 0x3FFEu);
+  if (i > total) return;
   Fused f{};
+  if (i == total) {  // the entry that serves no pc
+    f.w[7] = kNoRecord;
+    for (uint32_t j = 0; j < (uint32_t)kFusedWords / 4u; ++j)
+      fused[(size_t)i * (kFusedWords / 4) + j] = make_uint4(f.w[4 * j], f.w[4 * j + 1], f.w[4 * j + 2], f.w[4 * j + 3]);
+    return;
+  }
+  // A cart without bank switching has each window at a fixed address, so a
+  // JP's target is a place in the ROM (but not while the boot image is mapped)
+  const bool view = i >= rom_bytes + 0x4000u, fixed = rom_only != 0 && i < 0x8000u;
+  const uint32_t base = fixed ? 0u : i & ~0x3FFFu, k = i - base, lo = k & ~0x3FFFu;
+  const uint8_t* img = buf + base;
+  const uint32_t loops_from = view ? 0x100u : 0u;
+  const auto rec_of = [&](uint32_t at) { return record_at(img + (at & ~0x3FFFu), at & 0x3FFFu, loops_from); };
   FusedRun run{};
   run.main = k;
-  if (k < end) run = fused_run(img, k, lo, end, rom && abs_ok != 0);
-  const Rec nop = kDec.e[0];
+  if ((k & 0x3FFFu) < 0x3FFEu) run = fused_run(img, k, lo, lo + 0x3FFEu, fixed);
   for (uint32_t j = 0; j < kPure; ++j) {
-    Rec r = nop;
-    if (j < run.n) {
-      r = record_at(img, len, run.at[j], rom);
-      if ((r.w[0] & 0xFFu) == 0x18u || (r.w[0] & 0xFFu) == 0xC3u) r = nop;
-    }
-    pure_words(r, f.w + j * kPureWords);
+    const uint8_t* q = img + run.at[j];
+    if (j < run.n) pure_words(q[0], q[1], q[2], f.w + j * kPureWords);
+    else pure_words(0u, 0u, 0u, f.w + j * kPureWords);
   }
-  f.w[2] |= (run.main - k) << 16;
-  f.w[kPureWords + 2] |= (run.cycles | (run.n << 8)) << 16;
-  const Rec m = record_at(img, len, run.main, rom);
+  f.w[7] |= (k & 0x3FFFu) < 0x3FFEu ? (run.cycles | (run.n << 8)) << 16 : kNoRecord;
+  f.w[kPureWords + 7] |= (run.main - k) << 16;
+  const Rec m = rec_of(run.main), own = rec_of(k);
   for (int j = 0; j < kRecWords; ++j) f.w[kPure * kPureWords + j] = m.w[j];
   for (uint32_t j = 0; j < (uint32_t)kFusedWords / 4u; ++j)
     fused[(size_t)i * (kFusedWords / 4) + j] = make_uint4(f.w[4 * j], f.w[4 * j + 1], f.w[4 * j + 2], f.w[4 * j + 3]);
-  const Rec own = record_at(img, len, k, rom);
   for (uint32_t j = 0; j < (uint32_t)kRecWords / 4u; ++j)
     recs[(size_t)i * (kRecWords / 4) + j] = make_uint4(own.w[4 * j], own.w[4 * j + 1], own.w[4 * j + 2], own.w[4 * j + 3]);
 }
@@ -159,6 +162,13 @@ struct Ref32 {
   __device__ const Ref32& operator=(const Ref32& o) const { return *this = (int32_t)o; }
 };
 
+// Keeps the computation of the values in this block.
+__device__ __forceinline__ void pin1(uint32_t& v) { asm volatile("" : "+v"(v)); }
+template <typename... T>
+__device__ __forceinline__ void pin(T&... v) {
+  (pin1(v), ...);
+}
+__device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0F70); }  // vmcnt(0)
 __device__ __forceinline__ uint32_t sel(bool c, uint32_t a, uint32_t b) { return c ? a : b; }
 // c ? a : b for two computed addresses, marked unpredictable: left to
 // itself the compiler may turn such a select into a branch around the
@@ -213,7 +223,7 @@ struct Lane {
   const uint8_t* memb;             // memory image of the block (flat)
   const uint8_t* cramb;            // cartridge RAM of the block (flat)
   const uint8_t* rom;              // ROM buffer (flat)
-  uint32_t rom_len;
+  uint32_t rom_len, no_rec;
 
   // CPU: w0 = B C D E (B in bits 31-24), w1 = H L F A (A in bits 7-0)
   uint32_t pc, sp, w0, w1;
@@ -329,9 +339,12 @@ struct Lane {
     b0 = clamp_bank(b0, s.rom_banks, s.rom_mask);
     b1 = clamp_bank(b1, s.rom_banks, s.rom_mask);
     const int64_t lim = (int64_t)s.rom_banks * 0x4000;
-    // an unmapped bank reads the 0xFF filler that follows the boot image
-    const uint32_t open = rom_len + 0x100u;
+    // an unmapped bank reads the 0xFF window that follows the ROM
+    const uint32_t open = rom_len;
     rom_lo = ((int64_t)b0 * 0x4000 < lim) ? (uint32_t)b0 * 0x4000u : open;
+    // while the boot image is mapped, window 0 is the copy of the bank that
+    // has it in its first 256 bytes (banks 0, 32, 64 and 96 come here)
+    if (boot_en != 0u && rom_lo != open) rom_lo = rom_len + 0x4000u * (1u + ((uint32_t)b0 >> 5));
     rom_hi = ((int64_t)b1 * 0x4000 < lim) ? (uint32_t)b1 * 0x4000u : open;
     // (a runtime value even where cram rules RAM out: folded to a constant
     // it changed the compiler's schedule of the bus read, 1.7% slower)
@@ -350,8 +363,8 @@ struct Lane {
     rb = clamp_bank(rb, s.ram_banks, -1);
     const size_t blk = e >> kEnvBlockShift;
     const uint8_t* cb = cramb;
-    // nothing mapped: a byte of the 0xFF filler after the boot image
-    cart_p = rom + (rom_len + 0x100u);
+    // nothing mapped: a byte of the 0xFF window after the ROM
+    cart_p = rom + rom_len;
     cart_m = 0u;
     if (ram_ok && rtc_field >= 0) {
       const uint32_t slot = (uint32_t)(((mbr & kMbrLatch) ? CS_RTC_L_SECONDS : CS_RTC_SECONDS) + rtc_field);
@@ -382,11 +395,9 @@ struct Lane {
     const bool cart = x - 0xA000u < 0x2000u;
     // bitwise conditions throughout the per-instruction path: each is a
     // select, never a branch
-    const bool bootw = (boot_en != 0u) & (x < 0x100u);
-    const uint32_t win = (x < 0x4000u ? rom_lo : rom_hi) + (x & 0x3FFFu);
-    const uint32_t roff = win + ((rom_len + x - win) & (0u - (uint32_t)bootw));
+    const uint32_t roff = (x < 0x4000u ? rom_lo : rom_hi) + (x & 0x3FFFu);
     // (a cart without RAM never maps any)
-    const uint8_t* cp = cram ? cart_p + (((x - 0xA000u) << kEnvBlockShift) & cart_m) : this->rom + (rom_len + 0x100u);
+    const uint8_t* cp = cram ? cart_p + (((x - 0xA000u) << kEnvBlockShift) & cart_m) : this->rom + rom_len;
     const uint8_t* p = memb + ((x << kEnvBlockShift) | lane);
     p = cart ? cp : p;
     return sel_ptr(rom, this->rom + roff, p);
@@ -606,6 +617,7 @@ struct Lane {
         if (v != 0 && boot_en) {
           boot_en = 0;
           CS(CS_BOOTROM_ENABLED) = 0;
+          refresh_cart();  // window 0 no longer holds the boot image
           map_changed = 1;
         }
         break;
@@ -741,9 +753,9 @@ struct Lane {
   __device__ static bool plain_store(uint32_t x) { return plain_ram(x) | (x == 0xFF00u); }
   // The instruction's bus writes, in order (n = 0, 1 or 2).  When both are
   // plain stores they are stored without a branch; a lane with one write
-  // stores its first byte twice.  An MBC bank write clears rv, the validity
-  // of the record already fetched for the next pc (the boot ROM switch is an
-  // IO write, after which the full sequence drops the record).
+  // stores its first byte twice.  An MBC bank write makes the record already
+  // fetched for the next pc stale (the boot ROM switch is an IO write, after
+  // which the full sequence drops the record).
   // With cartridge RAM (cram), a byte of a mapped RAM bank is a plain store
   // too, into the cartridge RAM buffer instead of the env's memory.
   __device__ bool cart_plain(uint32_t x) const { return cram & (x - 0xA000u < 0x2000u) & (cart_m != 0u); }
@@ -753,7 +765,7 @@ struct Lane {
   }
   // `before` runs ahead of a write with side effects.
   template <typename F>
-  __device__ void write_bus(uint32_t n, uint32_t a0, uint32_t v0, uint32_t a1, uint32_t v1, bool& rv, F before) {
+  __device__ void write_bus(uint32_t n, uint32_t a0, uint32_t v0, uint32_t a1, uint32_t v1, uint32_t& stale, F before) {
     const uint32_t x0 = a0 & 0xFFFFu, x1 = a1 & 0xFFFFu;
     const bool two = n >= 2u;
     const bool c0 = cart_plain(x0), c1 = cart_plain(x1);
@@ -762,7 +774,7 @@ struct Lane {
       write8(a0, v0);
       if (two) write8(a1, v1);
       if (mbc != MBC_ROM_ONLY) {
-        rv = rv & (map_changed == 0u);
+        stale = map_changed != 0u ? 0xFFu : stale;
         map_changed = 0;
       }
     } else {
@@ -1175,24 +1187,13 @@ struct Lane {
 
   // -- fetch ---------------------------------------------------------------------
   // A pre-decoded record serves pc when all three instruction bytes lie in
-  // one 16 KiB ROM window of a mapped bank, or in the boot image.
-  __device__ bool rec_ok(uint32_t p) const {
-    const bool bw = (boot_en != 0u) & (p < 0x100u);
-    return (bw & (p < 0xFEu)) | (!bw & (p < 0x8000u) & ((p & 0x3FFFu) <= 0x3FFDu));
-  }
-  __device__ uint32_t rec_index(uint32_t p) const {
-    return ((boot_en != 0u) & (p < 0x100u)) ? rom_len + p
-                                   : (p < 0x4000u ? rom_lo : rom_hi) + (p & 0x3FFFu);
-  }
-  // rec_ok and rec_index in one: the record index for p, or 0 when no record
-  // serves it (ok false).  Written as selects so that the per-instruction
-  // path has no branch for it.
-  __device__ uint32_t next_rec(uint32_t p, bool& ok) const {
-    const bool bw = (boot_en != 0u) & (p < 0x100u);
-    const uint32_t win = sel(p < 0x4000u, rom_lo, rom_hi) + (p & 0x3FFFu);
-    ok = (bw & (p < 0xFEu)) | (!bw & (p < 0x8000u) & ((p & 0x3FFFu) <= 0x3FFDu));
-    return sel(ok, sel(bw, rom_len + p, win), 0u);
-  }
+  // one 16 KiB ROM window.
+  __device__ static bool rec_ok(uint32_t p) { return (p < 0x8000u) & ((p & 0x3FFFu) <= 0x3FFDu); }
+  __device__ uint32_t rec_index(uint32_t p) const { return (p < 0x4000u ? rom_lo : rom_hi) + (p & 0x3FFFu); }
+  // The index of the fused record for p: that of the entry that serves no pc
+  // above the ROM.  (The last two of each window say so themselves.)  Written
+  // as selects so that the per-instruction path has no branch for it.
+  __device__ uint32_t next_rec(uint32_t p) const { return sel(p < 0x8000u, sel(p < 0x4000u, rom_lo, rom_hi) + (p & 0x3FFFu), no_rec); }
   // Fetch + decode through the bus (code in RAM, window edges, open bus).
   __device__ Rec fetch_slow() const {
     const uint32_t b0 = read8(pc), b1 = read8(pc + 1u), b2 = read8(pc + 2u);
@@ -1226,6 +1227,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   L.cramb = in_vgpr(s.cram + (size_t)blk * (size_t)s.cram_stride * kEnvBlock);
   L.rom = in_vgpr(s.rom);
   L.rom_len = in_vgpr((uint32_t)s.rom_len);
+  L.no_rec = in_vgpr((uint32_t)s.no_rec);
   L.rsc = make_rsrc(s.sc + (size_t)blk * (kNumFields * kEnvBlock), kNumFields * kEnvBlock * 4);
   L.rcs = make_rsrc(s.cs + (size_t)blk * (kCartStateStride * kEnvBlock),
                     kCartStateStride * kEnvBlock * 4);
@@ -1314,14 +1316,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   constexpr bool dbg = kDbg;
 
   // record of the instruction at pc, with the pure instructions that run
-  // before it (valid when rv; the debug variants run every instruction alone)
+  // before it (the debug variants run every instruction alone)
   Rec rec{};
   uint32_t pure[kPure * kPureWords];
-  bool rv = false;
+  pure[7] = 0;
+  // 0xFF once something has made the loaded record stale
+  uint32_t stale = 0xFFu;
+  // Loads are kept in the order the words are used, and the rare block that
+  // loads a single record waits for it there (wait_loads): a pass then waits
+  // for each quad as it needs it and not, as at a join of the two paths, for
+  // every load and store in flight.
   auto ld_words = [&](const uint4* p, uint32_t* w, int quads) {
 #pragma unroll
     for (int k = 0; k < quads; ++k) {
       const u32x4 q = ld_global(reinterpret_cast<const u32x4*>(p + k));
+      asm volatile("" ::: "memory");
       w[4 * k] = q[0];
       w[4 * k + 1] = q[1];
       w[4 * k + 2] = q[2];
@@ -1330,27 +1339,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   };
   auto load_single = [&](uint32_t i) { ld_words(recs + (size_t)i * (kRecWords / 4), rec.w, kRecWords / 4); };
   auto load_rec = [&](uint32_t i) {
-    if (kDbg) {
-      load_single(i);
-    } else {
-      const uint4* p = fused + (size_t)i * (kFusedWords / 4);
-      ld_words(p, pure, kPure * kPureWords / 4);
-      ld_words(p + kPure * kPureWords / 4, rec.w, kRecWords / 4);
-    }
+    if (kDbg) return;
+    stale = 0;
+    const uint4* p = fused + (size_t)i * (kFusedWords / 4);
+    ld_words(p, pure, kPure * kPureWords / 4);
+    ld_words(p + kPure * kPureWords / 4, rec.w, kRecWords / 4);
   };
   // no pure instruction ahead of the record
   auto clear_pure = [&]() {
+    constexpr PureWords none = no_pure();
 #pragma unroll
-    for (uint32_t j = 0; j < kPure; ++j) {
-      uint32_t* p = pure + j * kPureWords;
-      p[0] = p[1] = kZero4;
-      p[2] = 0u;
-      p[3] = 0x03020100u;
-      p[4] = 0x03020000u | (U_FN << 8);
-      p[5] = FALL << 8;
-      p[6] = 9u | 0x0C0C0000u;
-      p[7] = 0x0C0Cu;
-    }
+    for (uint32_t j = 0; j < kPure * kPureWords; ++j) pure[j] = none.w[j % kPureWords];
   };
 
   // Block copies of the copy-loop fast-forward (bytes cp_src[j * cp_stride]
@@ -1428,24 +1427,26 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       // (rare branches of the per-instruction path test a wave-uniform
       // ballot first: when no lane takes them the path keeps its exec mask
       // instead of saving and restoring it around a skipped block)
-      if (!kDbg) cp = ubfe(pure[kPureWords + 2], 16, 8);
-      // no valid record, or an event within the pure instructions: the
-      // instruction at pc alone
-      const bool single = !rv | ((!kDbg) & (cp != 0u) & ((int)cp >= L.budget));
+      // no record, or an event within the pure instructions (there is none
+      // to run when cp is 0): the instruction at pc alone
+      cp = max(ubfe(pure[7], 16, 8), stale);
+      const bool single = kDbg | ((int)cp >= min(max(L.budget, 1), 0xFF));
       if (__builtin_expect(__ballot(single) != 0u, 0)) {
         if (single) {
           if (L.rec_ok(pc)) load_single(L.rec_index(pc));
           else rec = L.fetch_slow();
-          if (!kDbg) clear_pure();
+          clear_pure();
           cp = 0;
+          wait_loads();
         }
       }
+      uint32_t sph = L.sp << 16;
       if (!kDbg) {
-        exec_pure(pure, L.w0, L.w1, L.sp);
-        exec_pure(pure + kPureWords, L.w0, L.w1, L.sp);
-        pc = (pc + (pure[2] >> 16)) & 0xFFFFu;
+        exec_pure(pure, L.w0, L.w1, sph);
+        exec_pure(pure + kPureWords, L.w0, L.w1, sph);
+        pc = (pc + (pure[kPureWords + 7] >> 16)) & 0xFFFFu;
         pc_before = pc;
-        ninstr += pure[kPureWords + 2] >> 24;
+        ninstr += pure[7] >> 24;
       }
       op = rec.w[0] & 0xFFu;
       if (dbg) {  // debug traps before execution: the instruction does not run
@@ -1459,11 +1460,12 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       ExecIn in;
       in.w0 = L.w0;
       in.w1 = L.w1;
-      in.x1 = (L.sp << 16) | pc;
+      in.x1 = bit_select(0xFFFF0000u, sph, pc);
       in.ra = operand_address(rec, L.w0, L.w1, in.x1);
 
       // ---- bus reads ------------------------------------------------------------
       const uint32_t nr = ubfe(rec.w[7], 8, 2);
+      ExecPre pre;
       {
         // Every lane loads the byte at its operand address, reading or not
         // (a read has no side effect, and the folded address is always on
@@ -1475,6 +1477,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
         const uint32_t x0 = Lane::fold(in.ra);
         const uint8_t* p0 = L.bus_ptr(x0);
         const uint32_t v0 = ld_global(p0);
+        // (pinned here: the load's latency covers them)
+        pre = exec_before_read(rec, in.w0, in.w1, in.x1, in.ra);
+        pin(pre.xy, pre.ab, pre.ci, pre.mor, pre.mand, pre.vw);
+        pin(pre.seq, pre.taken, pre.sel, pre.sp, pre.wa);
         uint32_t x1 = x0, v1 = 0;
         if (__builtin_expect(nr > 1u, 0)) {
           x1 = Lane::fold(in.ra + 1u);
@@ -1484,22 +1490,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
           v1 = ld_global(p1);
         }
         // DIV, TIMA, STAT and LY (FF04 FF05 FF40 FF41 FF44 FF45, bus_fix's
-        // test) for both bytes behind one wave-uniform test, the bytes
-        // taken by selects
-        const bool h0 = (nr != 0u) & ((x0 & 0xFFBAu) == 0xFF00u) & (x0 > 0xFF01u);
-        const bool h1 = (nr > 1u) & ((x1 & 0xFFBAu) == 0xFF00u) & (x1 > 0xFF01u);
-        uint32_t r0 = v0, r1 = v1;
-        if (__builtin_expect(__ballot(h0 | h1) != 0u, 0)) {
+        // test) for both bytes behind one wave-uniform test: any of them puts
+        // the first byte's address into FF02-FF45.  (An instruction without
+        // reads has no use for either byte.)
+        in.rd0 = v0;
+        in.rd1 = v1;
+        if (__builtin_expect(__ballot(x0 - 0xFF02u < 0x44u) != 0u, 0)) {
+          const bool h0 = (nr != 0u) & ((x0 & 0xFFBAu) == 0xFF00u) & (x0 > 0xFF01u);
+          const bool h1 = (nr > 1u) & ((x1 & 0xFFBAu) == 0xFF00u) & (x1 > 0xFF01u);
           if (h0 | h1) count_pure();
-          r0 = h0 ? L.read_ppu(x0, v0) : v0;
-          r1 = h1 ? L.read_ppu(x1, v1) : v1;
+          in.rd0 = h0 ? L.read_ppu(x0, v0) : v0;
+          in.rd1 = h1 ? L.read_ppu(x1, v1) : v1;
         }
-        in.rd0 = nr != 0u ? r0 : 0u;
-        in.rd1 = nr > 1u ? r1 : in.rd0;
       }
 
       // ---- execute (gbx_exec.h) -------------------------------------------------
-      const ExecOut o = exec_insn(rec, in);
+      const ExecOut o = exec_after_read(rec, in, pre);
       L.w0 = o.w0;
       L.w1 = o.w1;
       L.sp = o.sp;
@@ -1513,24 +1519,25 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       // (a wave-uniform test, so that the copy below runs with every lane
       // that is executing an instruction)
       if (__builtin_expect(__ballot(o.misc != 0u) != 0u, 0)) {
-        if (o.misc != 0u) {  // DI EI RETI HALT, illegal opcodes, poll/copy loops
+        if (o.misc != 0u) {  // DI EI RETI HALT DAA, illegal opcodes, poll/copy loops
           count_pure();
           L.settle();  // the fast-forwards start from the PPU and timer state
-          if (o.misc & 1u) {
-            L.ime = (o.misc >> 1) & 1u;
+          if (o.misc & kMiscIme) {
+            L.ime = o.misc & kMiscImeOn ? 1u : 0u;
             L.ime_delay = 0;
           }
-          if (o.misc & 4u) L.halted = 1;
+          if (o.misc & kMiscDaa) L.w1 = exec_daa(in.w1);
+          if (o.misc & kMiscHalt) L.halted = 1;
           // the step's interrupt check services or wakes on a pending request
           if (((L.ime | L.halted) != 0u) & ((L.ie & L.ifr & 0x1Fu) != 0u)) L.budget = 0;
-          if (o.misc & 8u) {  // misc.py:42-56: freeze the env, pc unchanged
+          if (o.misc & kMiscTrap) {  // misc.py:42-56: freeze the env, pc unchanged
             trap = 1;
             trap_pc = (int)pc;
             trap_op = (int)op;
             trap_kind = 1;
             L.budget = 0;
           }
-          if (!dbg && (o.misc & 16u) && (rec.w[15] & kCopyLoop)) {
+          if (!dbg && (o.misc & kMiscLoop) && (rec.w[15] & kCopyLoop)) {
             // LD A,(HL+) of a block-copy loop just ran: advance k whole passes
             // (this LD included) in one step.  Each pass copies (HL+) to (DE)
             // and steps DE and BC; OR leaves Z clear (BC stays non-zero), N,
@@ -1551,7 +1558,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
               rtc_pre = cycles - 12;
               ninstr += 7u * (uint32_t)k - 1u;
             }
-          } else if (!dbg && (o.misc & 16u)) {
+          } else if (!dbg && (o.misc & kMiscLoop)) {
             // The load of an LY poll loop just read LY into A; if CP d8 and the
             // jump take it back, every pass until LY or anything else can
             // change reads the same LY and leaves the same A and F: advance k
@@ -1592,7 +1599,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       }
       L.pc = npc;
       // fetch the next record while the writes, timer and PPU run
-      load_rec(L.next_rec(npc, rv));
+      load_rec(L.next_rec(npc));
       }
     } else {
       L.settle();
@@ -1602,7 +1609,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
 
     // ---- write phase, debug checks, timer, PPU, interrupt check --------------
     int svc = 0;
-    if (__builtin_expect(wn != 0u, 1)) L.write_bus(wn, wa0, wv0, wa1, wv1, rv, count_pure);
+    if (__builtin_expect(wn != 0u, 1)) L.write_bus(wn, wa0, wv0, wa1, wv1, stale, count_pure);
     if (dbg) {
       if (!hiter) {
         if (dbg_rst38 && L.pc >= 0xFE00u && !trap) {
@@ -1665,18 +1672,18 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
             L.write8((L.sp - k) & 0xFFFFu, k == 1 ? ret >> 8 : ret & 0xFFu);
           L.sp = (L.sp - 2u) & 0xFFFFu;
           L.pc = 0x40u + 8u * (uint32_t)__builtin_ctz(bit);
-          rv = false;
+          stale = 0xFFu;
           svc = 20;
           L.timer_tick(20);
           lcdc_now = L.ppu_advance(20);
         } else if (hiter) {
           L.pc = (L.pc + 1u) & 0xFFFFu;  // IME=0 wake skips a byte
-          rv = false;
+          stale = 0xFFu;
         }
       }
       if (__builtin_expect(L.map_changed != 0u, 0)) {
         L.map_changed = 0;
-        rv = false;
+        stale = 0xFFu;
       }
 
       const int total = cycles + svc;
@@ -1806,9 +1813,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
 
 }  // namespace
 
-hipError_t launch_build_records(const DevState& s, int64_t total, hipStream_t st) {
-  hipLaunchKernelGGL(build_records_kernel, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, st, s.rom,
-                     (uint32_t)s.rom_len, (uint32_t)total, s.mbc_kind == MBC_ROM_ONLY ? 1 : 0,
+hipError_t launch_build_records(const DevState& s, hipStream_t st) {
+  hipLaunchKernelGGL(build_records_kernel, dim3((unsigned)(s.no_rec / 256 + 1)), dim3(256), 0, st, s.rom,
+                     (uint32_t)s.rom_len, (uint32_t)s.no_rec, s.mbc_kind == MBC_ROM_ONLY ? 1 : 0,
                      const_cast<uint4*>(s.recs), const_cast<uint4*>(s.fused));
   return hipGetLastError();
 }

@@ -70,23 +70,23 @@ void harness_exec(const uint32_t* in, uint32_t* out) {
   e.ra = gbx::operand_address(r, e.w0, e.w1, e.x1);
   const gbx::ExecOut o = gbx::exec_insn(r, e);
   const uint32_t res[12] = {e.ra, o.w0, o.w1, o.sp, o.npc, o.cycles, o.wn, o.wa0,
-                            o.wv0, o.wa1, o.wv1, o.misc};
+                            o.wv0, o.wa1, o.wv1, gbx::ubfe(o.misc, 24, 5)};
   for (int k = 0; k < 12; ++k) out[k] = res[k];
 }
 
 // out: [is pure, its eight words]
 void harness_pure_words(uint32_t op, uint32_t b1, uint32_t b2, uint32_t* out) {
   out[0] = gbx::pure_op(op, b1) ? 1u : 0u;
-  gbx::pure_words(gbx::decode_insn(op, b1, b2), out + 1);
+  if (out[0]) gbx::pure_words(op, b1, b2, out + 1);
 }
 
 // in: pure words[8], w0, w1, sp (11 words); out: w0, w1, sp
 void harness_pure(const uint32_t* in, uint32_t* out) {
-  uint32_t w0 = in[8], w1 = in[9], sp = in[10];
-  gbx::exec_pure(in, w0, w1, sp);
+  uint32_t w0 = in[8], w1 = in[9], sph = in[10] << 16;
+  gbx::exec_pure(in, w0, w1, sph);
   out[0] = w0;
   out[1] = w1;
-  out[2] = sp & 0xFFFFu;
+  out[2] = sph >> 16;
 }
 
 // out: [number of pure instructions, cycles, main offset, their offsets]

@@ -183,25 +183,30 @@ int parse_header(const uint8_t* rom, int64_t rom_len, int* kind, int64_t* rom_by
 }
 
 // Envs per step-kernel wavefront.  Each env is a serial instruction stream,
-// so a wavefront's time per emulated instruction is set by its dependent
-// memory round trips, not by how many lanes it carries.  Below ~4 wavefronts
-// per CU some SIMDs would sit idle, so small env counts are spread over
-// narrower workgroups (64 -> 32 -> 16 -> 8 envs) until every SIMD holds one.
+// and a pass of the loop costs a wavefront about the same however many lanes
+// it carries; what slows it down is company on its CU (and on the CU that
+// shares its instruction cache).  So a wavefront takes a whole 64-env block,
+// and 16,384 envs are one wavefront per CU: random-code cart, frameskip 4, at
+// 8,192 / 16,384 / 32,768 envs 10.7 / 10.7 / 11.8 ms with 64 envs a wavefront,
+// 12.3 / 11.2 / 12.5 with 32, 18.0 / 11.4 / 15.9 with 16.  Carts with a bank
+// controller run interrupt and halt handling in which each lane delays the
+// others: while it still gives every CU at most one wavefront, 8 envs a
+// wavefront are faster (MBC1 at 64 / 2,048 envs 4.4 / 4.6 ms against 5.1 / 5.4
+// with 64; at 4,096 envs they are level).
 // GBX_STEP_LANES=64|32|16|8|4 overrides the choice (for tuning sweeps).
-int choose_step_lanes(int n) {
+int choose_step_lanes(int n, int kind, int cus) {
   if (const char* v = getenv("GBX_STEP_LANES")) {
     const int l = atoi(v);
     if (l == 4 || l == 8 || l == 16 || l == 32 || l == 64) return l;
   }
-  int dev = 0, cus = 256;
-  if (hipGetDevice(&dev) == hipSuccess) {
-    int x = 0;
-    if (hipDeviceGetAttribute(&x, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && x > 0)
-      cus = x;
-  }
-  int lanes = kEnvBlock;
-  while (lanes > 8 && (n + lanes - 1) / lanes < 4 * cus) lanes >>= 1;
-  return lanes;
+  return kind != MBC_ROM_ONLY && (n + 7) / 8 <= cus ? 8 : kEnvBlock;
+}
+int cu_count() {
+  int dev = 0, x = 0;
+  if (hipGetDevice(&dev) == hipSuccess &&
+      hipDeviceGetAttribute(&x, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && x > 0)
+    return x;
+  return 256;
 }
 
 // Envs [env_lo, env_hi) x addresses [lo, hi) inside the context.
@@ -249,7 +254,14 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   s.cram_stride = ram_bytes > 0 ? ram_bytes : 1;
   s.mbc_kind = kind;
   s.rom_len = rom_bytes;
-  s.step_lanes = choose_step_lanes(num_envs);
+  const int cus = cu_count();
+  s.step_lanes = choose_step_lanes(num_envs, kind, cus);
+  // One wavefront to a workgroup, except for carts with a bank controller and
+  // RAM once CUs hold several: their wavefronts run better four to a CU on
+  // half of the CUs (MBC3, frameskip 4, 32,768 / 49,152 envs: 8.5 / 8.5 ms
+  // against 9.3 / 9.4; level from 65,536 on, and 8.8 against 8.0 at 16,384).
+  s.step_threads = s.step_lanes == kEnvBlock && kind != MBC_ROM_ONLY && ram_bytes > 0 && s.npad / kEnvBlock > cus
+                       ? 4 * kEnvBlock : s.step_lanes;
   const size_t np = (size_t)s.npad;
   hipError_t e = hipSuccess;
   auto A = [&](hipError_t r) {

@@ -95,7 +95,8 @@ struct DevState {
   const uint4* fused;       // fused record (pure instructions and the one after them) per byte
   int n, npad, obs_dim;
   int rom_banks, rom_mask, ram_banks, ram_bytes, cram_stride, mbc_kind;
-  int step_lanes;       // envs per step-kernel wavefront: 64, 32, 16 or 8
+  int step_lanes;       // envs per step-kernel wavefront: 64, 32, 16, 8 or 4
+  int step_threads;     // threads of its workgroups: step_lanes, or 256
   int64_t rom_len;
   int64_t no_rec;       // bytes of the ROM buffer, the fused record that serves no pc
 };

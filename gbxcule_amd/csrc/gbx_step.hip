@@ -1206,10 +1206,9 @@ struct Lane {
 // ---------------------------------------------------------------------------
 // One variant per cartridge kind (kMbc), per debug mode (kDbg) and, for
 // ROM-only carts, per declared RAM (kCram): the cartridge code of other
-// kinds and every debug check compile out.  The variants for MBC carts
-// with RAM are built for two wavefronts per SIMD (256 VGPRs): at three they
-// spill VGPRs to scratch in the loop, and 131,072 envs in 64-lane
-// wavefronts are two per SIMD.
+// kinds and every debug check compile out.  Built for two wavefronts per SIMD
+// (256 VGPRs, about 200 used): 131,072 envs in 64-lane wavefronts are two per
+// SIMD.
 template <int kMbc, bool kDbg, bool kCram = true>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void step_kernel(DevState s, StepArgs args) {
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1823,12 +1822,8 @@ hipError_t launch_build_records(const DevState& s, hipStream_t st) {
 hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st) {
   if (s.n <= 0) return hipSuccess;
   // A wavefront carries step_lanes envs (a divisor of the 64-env memory
-  // block, so it never straddles two blocks).  Full 64-lane wavefronts go
-  // four to a workgroup: the four land on the four SIMDs of one CU, where
-  // single-wavefront workgroups left some SIMDs with three wavefronts and
-  // others with one (the wavefronts on a crowded SIMD set the launch time).
-  // Narrower wavefronts (few envs) stay one to a workgroup, one per SIMD.
-  const int threads = s.step_lanes == kEnvBlock ? 4 * kEnvBlock : s.step_lanes;
+  // block, so it never straddles two blocks).
+  const int threads = s.step_threads;
   const int blocks = (s.n + threads - 1) / threads;
   const bool dbg = a.dbg_rst38 || a.dbg_trap_pc || a.dbg_max_instr > 0 || a.dbg_watch;
   const dim3 g(blocks), b(threads);

@@ -57,6 +57,8 @@ SIGNATURES: dict[str, tuple[object, list[object]]] = {
     "gbx_write_mem": (ctypes.c_int, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
     "gbx_state_hash": (ctypes.c_int, [_vp, _vp, _vp]),
     "gbx_export_scalar": (ctypes.c_int, [_vp, _i32, _vp]),
+    "gbx_export_scalars": (ctypes.c_int, [_vp, _i32, _vp]),
+    "gbx_packed_l1": (ctypes.c_int, [_vp, _i64, _vp, _i64, _i64, _i64, ctypes.c_float, _vp, _vp]),
     "gbx_import_scalar": (ctypes.c_int, [_vp, _i32, _vp]),
     "gbx_export_mem": (ctypes.c_int, [_vp, _i32, _i32, _i32, _i32, _vp]),
     "gbx_import_mem": (ctypes.c_int, [_vp, _i32, _i32, _vp, _i32]),

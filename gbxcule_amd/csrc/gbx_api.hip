@@ -483,6 +483,39 @@ int gbx_export_scalar(gbx_ctx* ctx, int32_t field, int64_t* host_out) {
   return GBX_OK;
 }
 
+int gbx_export_scalars(gbx_ctx* ctx, int32_t env, int64_t* scalars) {
+  CHECK_CTX(ctx);
+  if (!scalars) return fail(GBX_E_INVALID, "out is NULL");
+  if (env < 0 || env >= ctx->s.n) return fail(GBX_E_INVALID, "env out of range");
+  const DevState& s = ctx->s;
+  // the env's 64-env block of every field (8 KiB) and counter (1 KiB)
+  int32_t sc[kNumFields * kEnvBlock];
+  int64_t cnt[2 * kEnvBlock];
+  int32_t action = 0;
+  const size_t blk = (size_t)env >> kEnvBlockShift;
+  const uint32_t lane = (uint32_t)env & (kEnvBlock - 1);
+  HIP_TRY(hipDeviceSynchronize());
+  HIP_TRY(hipMemcpy(sc, s.sc + blk * (kNumFields * kEnvBlock), sizeof(sc), hipMemcpyDeviceToHost));
+  HIP_TRY(hipMemcpy(cnt, s.cnt + blk * (2 * kEnvBlock), sizeof(cnt), hipMemcpyDeviceToHost));
+  HIP_TRY(hipMemcpy(&action, s.actions + env, sizeof(action), hipMemcpyDeviceToHost));
+  for (int f = 0; f < kNumFields; ++f) scalars[f] = sc[sc_index(lane, f)];
+  scalars[F_INSTR] = cnt[cnt_index(lane, 0)];
+  scalars[F_CYCLES] = cnt[cnt_index(lane, 1)];
+  scalars[F_ACTIONS] = action;
+  return GBX_OK;
+}
+
+int gbx_packed_l1(const uint8_t* obs_dev, int64_t obs_stride, const uint8_t* goal_dev, int64_t goal_stride, int64_t n,
+                  int64_t bytes, float scale, float* out_dev, void* stream) {
+  // (a frame's sum, at most 12 per byte, stays in 32 bits)
+  if (n < 0 || bytes < 0 || bytes > (1 << 26) || n > (int64_t)INT32_MAX * 4)
+    return fail(GBX_E_INVALID, "frame count or size out of range");
+  if (n == 0) return GBX_OK;
+  if (!out_dev || (bytes > 0 && (!obs_dev || !goal_dev))) return fail(GBX_E_INVALID, "frames or output NULL");
+  HIP_TRY(launch_packed_l1(obs_dev, obs_stride, goal_dev, goal_stride, n, bytes, scale, out_dev, (hipStream_t)stream));
+  return GBX_OK;
+}
+
 int gbx_import_scalar(gbx_ctx* ctx, int32_t field, const int64_t* host_in) {
   CHECK_CTX(ctx);
   if (!host_in) return fail(GBX_E_INVALID, "in is NULL");

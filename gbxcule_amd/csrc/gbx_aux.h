@@ -49,6 +49,8 @@ struct HashTable {
 };
 constexpr size_t kHashDigits = (size_t)kMemSize * 16;
 hipError_t launch_hash(const DevState& s, const HashTable& k, uint64_t* out, hipStream_t st);
+hipError_t launch_packed_l1(const uint8_t* obs, int64_t obs_stride, const uint8_t* goal, int64_t goal_stride,
+                            int64_t n, int64_t bytes, float scale, float* out, hipStream_t st);
 // buf[count][len] env-major <-> memory of envs [env_lo, env_lo + count),
 // addresses [lo, lo + len); to_image = 0 reads the image into buf, 1 writes
 // buf into the image.  The caller checks the ranges.

@@ -68,6 +68,62 @@ def get_diff_lut(device=None):
     return lut
 
 
+def _frame_stride(t):
+    """Bytes from one frame to the next of a CUDA tensor [N, 1, H, W_bytes]
+    whose frames are contiguous, else None."""
+    n, _, h, w = t.shape
+    if (w > 1 and t.stride(3) != 1) or (h > 1 and t.stride(2) != w):
+        return None
+    return int(t.stride(0)) if n > 1 else h * w
+
+
+def _l1_kernel_operands(obs, goal):
+    """(obs stride, goal stride) when the distance kernel may take the frames:
+    plain CUDA tensors of one device, the current one, outside tracing,
+    function transforms and dispatch modes, which have to see torch calls."""
+    torch = _torch()
+    if type(obs) is not torch.Tensor or type(goal) is not torch.Tensor or not (obs.is_cuda and goal.is_cuda):
+        return None
+    if obs.device != goal.device or obs.device.index != torch.cuda.current_device():
+        return None
+    if obs.shape[1] != 1 or obs.numel() == 0 or obs.shape[2] * obs.shape[3] > 1 << 26:
+        return None
+    if (
+        torch.jit.is_tracing()
+        or torch.compiler.is_compiling()
+        or torch._C._len_torch_dispatch_stack() > 0
+        or torch._C._len_torch_function_stack() > 0
+        or torch._C._functorch.peek_interpreter_stack() is not None
+    ):
+        return None
+    strides = _frame_stride(obs), _frame_stride(goal)
+    if None in strides:
+        return None
+    return strides[0], 0 if goal.shape[0] == 1 else strides[1]
+
+
+def _l1_kernel(obs, obs_stride, goal, goal_stride):
+    """One launch for the whole distance (the torch form below is about 25).
+    Scaled by the 32-bit reciprocal, as torch divides by a number on the GPU."""
+    torch = _torch()
+    import ctypes
+
+    import numpy as np
+
+    from .. import _lib
+
+    n, _, h, w = obs.shape
+    out = torch.empty((n,), dtype=torch.float32, device=obs.device)
+    scale = float(np.float32(1.0) / np.float32(h * w * 4 * 3))
+    _lib.check(
+        _lib.load().gbx_packed_l1(
+            ctypes.c_void_p(obs.data_ptr()), obs_stride, ctypes.c_void_p(goal.data_ptr()), goal_stride, n, h * w,
+            scale, ctypes.c_void_p(out.data_ptr()), ctypes.c_void_p(int(torch.cuda.current_stream().cuda_stream)),
+        )
+    )  # fmt: skip
+    return out
+
+
 def packed_l1_distance(packed_obs, packed_goal):
     """Mean per-pixel shade distance to a goal, in [0, 1]: sum |obs - goal| over
     the 4 x H x W_bytes pixels of each env, divided by 3 x pixels
@@ -99,6 +155,9 @@ def packed_l1_distance(packed_obs, packed_goal):
             f"packed_goal: {goal.shape[0]} goals for {packed_obs.shape[0]} observations (expected 1 or N)"
         )
     packed_goal = goal
+    strides = _l1_kernel_operands(packed_obs, goal)
+    if strides is not None:
+        return _l1_kernel(packed_obs, strides[0], goal, strides[1])
     o = packed_obs.to(torch.int16)
     g = packed_goal.to(torch.int16)
     d = torch.zeros_like(o)

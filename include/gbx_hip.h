@@ -147,11 +147,24 @@ int gbx_write_mem(gbx_ctx* ctx, int32_t env_lo, int32_t env_hi, int32_t lo,
  * counterpart: lets callers compare full state without a readback). */
 int gbx_state_hash(gbx_ctx* ctx, uint64_t* out_dev, void* stream);
 
+/* out_dev[i] = (sum over the frame's pixels of |obs - goal|) * scale for n
+ * packed frames of `bytes` bytes (four 2-bit shades each); goal_stride 0: one
+ * goal for all, `bytes`: one per frame, and obs_stride the bytes from one
+ * frame to the next (rl/packed_metrics.py:16-41).  No context: any packed
+ * frames on the current device. */
+int gbx_packed_l1(const uint8_t* obs_dev, int64_t obs_stride, const uint8_t* goal_dev,
+                  int64_t goal_stride, int64_t n, int64_t bytes, float scale,
+                  float* out_dev, void* stream);
+
 /* Synchronous readback / writeback helpers (get_cpu_state 947-1009,
  * read_memory 766-797, get_cart_state 1011-1022, read_serial 1409-1431,
  * write_memory 899-911 of backends/warp_vec.py). */
 int gbx_export_scalar(gbx_ctx* ctx, int32_t field, int64_t* host_out);
 int gbx_import_scalar(gbx_ctx* ctx, int32_t field, const int64_t* host_in);
+/* One env's scalars[GBX_NUM_FIELDS] (GBX_FIELD_* order), for callers that
+ * read one env's registers (get_cpu_state): the same values as
+ * gbx_export_scalar of every field, without copying every env's. */
+int gbx_export_scalars(gbx_ctx* ctx, int32_t env, int64_t* scalars);
 int gbx_export_mem(gbx_ctx* ctx, int32_t env_lo, int32_t env_hi, int32_t lo,
                    int32_t hi, uint8_t* host_out);
 /* gbx_import_mem and gbx_import_env write the rows the step never writes

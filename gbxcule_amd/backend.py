@@ -622,7 +622,9 @@ class HipVecBackend:
             raise RuntimeError("Backend not initialized. Call reset() first.")
         names = ("pc", "sp", "a", "f", "b", "c", "d", "e", "h", "l", "instr_count",
                  "cycle_count", "trap_flag", "trap_pc", "trap_opcode", "trap_kind")  # fmt: skip
-        st = {n: int(self.export_field(n)[env_idx]) for n in names}
+        vals = np.empty((len(_lib.FIELDS),), dtype=np.int64)
+        self._call("gbx_export_scalars", self.ctx, env_idx, vals.ctypes.data_as(ctypes.c_void_p))
+        st = {n: int(vals[_lib.FIELD_ID[n]]) for n in names}
         st["pc"] &= 0xFFFF
         st["sp"] &= 0xFFFF
         for r in "abcdehl":

@@ -282,13 +282,13 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   A(dalloc(&s.frame_bg, (size_t)kScreenW * kScreenH));
   uint8_t *drom = nullptr, *dboot = nullptr;
   Rec* drecs = nullptr;
-  Fused* dfused = nullptr;
+  uint32_t* dfused = nullptr;
   const std::vector<uint8_t> rombuf = rom_buffer(rom, rom_bytes, boot, kind);
   s.no_rec = (int64_t)rombuf.size();
   A(dalloc(&drom, rombuf.size()));
   A(dalloc(&dboot, (size_t)0x100));
   A(dalloc(&drecs, rombuf.size()));
-  A(dalloc(&dfused, rombuf.size() + 1));
+  A(dalloc(&dfused, (rombuf.size() + 1) * kFusedStride));
   s.rom = drom;
   s.boot = dboot;
   s.recs = reinterpret_cast<const uint4*>(drecs);

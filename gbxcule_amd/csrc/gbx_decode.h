@@ -558,13 +558,16 @@ __host__ __device__ constexpr Rec decode_insn(uint32_t op, uint32_t b1, uint32_t
 // ADD HL,rr and the SP forms are left out: they alone take flags from the
 // 16-bit adder, whose carries then need no instructions here.
 // ---------------------------------------------------------------------------
-constexpr uint32_t kPure = 2;
+constexpr uint32_t kPure = 4;
+constexpr uint32_t kPureFirst = 2;  // of them in the record's first 128-byte line
 constexpr int kPureWords = 8;
 constexpr int kFusedWords = kPure * kPureWords + kRecWords;
+constexpr int kFusedStride = 64;  // words from one fused record to the next: two 128-byte lines
 // In p7 of the first: no record here (more cycles than any run has).
 constexpr uint32_t kNoRecord = 0xFFu << 16;
 struct Fused {
-  uint32_t w[kFusedWords];  // pure instructions, then the main record
+  // the first kPureFirst pure instructions, the main record, the others
+  uint32_t w[kFusedWords];
 };
 __host__ __device__ constexpr bool pure_op(uint32_t op, uint32_t b1) {
   const uint32_t z = op & 7u, y = (op >> 3) & 7u, p = op >> 4;

@@ -33,13 +33,19 @@ __device__ __forceinline__ uint32_t bit_mask(uint32_t w) {
   asm("v_bfe_i32 %0, %1, %2, 1" : "=v"(r) : "v"(w), "i"(pos));
   return r;
 }
+// bits of a where the constant m is set, of b elsewhere: V_BFI_B32 (left as
+// masks the compiler spends three instructions on each)
+template <uint32_t m>
+__device__ __forceinline__ uint32_t bit_select(uint32_t a, uint32_t b) {
+  uint32_t r;
+  asm("v_bfi_b32 %0, %1, %2, %3" : "=v"(r) : "s"(m), "v"(a), "v"(b));
+  return r;
+}
 // per-16-bit-half add, each half wrapping
 __device__ __forceinline__ uint32_t add_u16x2(uint32_t a, uint32_t b) {
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(gbx_u16x2, a) + __builtin_bit_cast(gbx_u16x2, b));
 }
 #endif
-// bits of a where m is set, of b elsewhere (V_BFI_B32)
-__device__ __forceinline__ uint32_t bit_select(uint32_t m, uint32_t a, uint32_t b) { return (a & m) | (b & ~m); }
 
 struct ExecIn {
   uint32_t w0, w1;     // register file: B C D E / H L F A
@@ -188,13 +194,14 @@ __device__ __forceinline__ void exec_pure(const uint32_t* p, uint32_t& w0, uint3
   // H in bit 4 and C in bit 8: carries, borrows when y was complemented
   // (y itself takes part here, and bit 8 of the mask inverts the last carry)
   const uint32_t fs = (s9 ^ x ^ y) | perm(W1, XYA, p[1]);
-  const uint32_t nhc = bit_select(0x6000u, (fs << 9) | 0x4000u, fs << 4);
-  const uint32_t fw = bit_select(0x8000u, res - 1u, nhc);  // Z: res - 1 wraps
+  const uint32_t nhc = bit_select<0x6000u>((fs << 9) | 0x4000u, fs << 4);
+  const uint32_t fw = bit_select<0x8000u>(res - 1u, nhc);  // Z: res - 1 wraps
   const uint32_t f = (fw & p[5]) | (W1 & p[7]);
-  const uint32_t U = bit_select(0xFFu, res, bit_select(0xFFFF0000u, sum, f));
+  const uint32_t U = bit_select<0xFFu>(res, bit_select<0xFFFF0000u>(sum, f));
   w0 = perm(U, W0, p[3]);
   w1 = perm(U, W1, p[4]);
-  sph = bit_select(bit_mask<7>(p[2]), sum, sph);
+  const uint32_t mspw = bit_mask<7>(p[2]);
+  sph = (sum & mspw) | (sph & ~mspw);
 }
 
 }  // namespace gbx

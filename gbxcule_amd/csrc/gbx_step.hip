@@ -10,16 +10,17 @@
 // The implementation is not a translation of that kernel.  A wavefront runs
 // up to 64 independent instruction streams, so the loop body is built to
 // cost the same whatever mix of opcodes its lanes execute:
-//  * fetch + decode is eight 16-byte loads of the pre-decoded 128-byte fused
-//    record at pc (gbx_decode.h), issued for the next pc while the current
-//    instruction's writes, timer and PPU work run.  One pass of the loop runs
-//    the record's up to two register-only instructions and the instruction
-//    after them: bus address, read latency, write phase and timer are paid
-//    once for all (2.2-2.4 instructions a pass on the random-code carts, for
-//    about 75 more VALU instructions; 16,384 envs, frameskip 24: 128.0 -> 85.4
-//    ms; 64 envs, frameskip 4: 29.7 -> 17.4 ms).  Two, since a third finds a
-//    register-only instruction in few passes only, and two fill one 128-byte
-//    line.  A pass whose register-only instructions would reach an event
+//  * fetch + decode is eight 16-byte loads of the first line of the
+//    pre-decoded fused record at pc (gbx_decode.h), issued for the next pc
+//    while the current instruction's writes, timer and PPU work run.  One pass
+//    of the loop runs the record's up to four register-only instructions and
+//    the instruction after them: bus address, read latency, write phase and
+//    timer are paid once for all, for 37 VALU instructions each (2.7-3.1
+//    instructions a pass on the random-code carts).  Two of them are in the
+//    first line; the others cost a pass nothing where no lane has them.  With
+//    none / two / four, same launch shape for the last two: 16,384 envs
+//    frameskip 24 128.0 / 71.9 / 67.7 ms, 64 envs frameskip 4 29.7 / 13.9 /
+//    11.9 ms.  A pass whose register-only instructions would reach an event
 //    (event_budget) runs the instruction at pc alone;
 //  * what an instruction computes without the bytes it reads (carry-in,
 //    branch, SP, write addresses) is pinned behind the issue of the read,
@@ -94,10 +95,15 @@ __global__ void build_records_kernel(const uint8_t* buf, uint32_t rom_bytes, uin
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > total) return;
   Fused f{};
-  if (i == total) {  // the entry that serves no pc
-    f.w[7] = kNoRecord;
+  const auto store_fused = [&]() {
     for (uint32_t j = 0; j < (uint32_t)kFusedWords / 4u; ++j)
-      fused[(size_t)i * (kFusedWords / 4) + j] = make_uint4(f.w[4 * j], f.w[4 * j + 1], f.w[4 * j + 2], f.w[4 * j + 3]);
+      fused[(size_t)i * (kFusedStride / 4) + j] = make_uint4(f.w[4 * j], f.w[4 * j + 1], f.w[4 * j + 2], f.w[4 * j + 3]);
+  };
+  const auto pure_at = [&](uint32_t j) { return f.w + (j < kPureFirst ? j * kPureWords : kRecWords + j * kPureWords); };
+  if (i == total) {  // the entry that serves no pc
+    for (uint32_t j = 0; j < kPure; ++j) pure_words(0u, 0u, 0u, pure_at(j));
+    f.w[7] |= kNoRecord;
+    store_fused();
     return;
   }
   // A cart without bank switching has each window at a fixed address, so a
@@ -112,15 +118,14 @@ __global__ void build_records_kernel(const uint8_t* buf, uint32_t rom_bytes, uin
   if ((k & 0x3FFFu) < 0x3FFEu) run = fused_run(img, k, lo, lo + 0x3FFEu, fixed);
   for (uint32_t j = 0; j < kPure; ++j) {
     const uint8_t* q = img + run.at[j];
-    if (j < run.n) pure_words(q[0], q[1], q[2], f.w + j * kPureWords);
-    else pure_words(0u, 0u, 0u, f.w + j * kPureWords);
+    if (j < run.n) pure_words(q[0], q[1], q[2], pure_at(j));
+    else pure_words(0u, 0u, 0u, pure_at(j));
   }
   f.w[7] |= (k & 0x3FFFu) < 0x3FFEu ? (run.cycles | (run.n << 8)) << 16 : kNoRecord;
   f.w[kPureWords + 7] |= (run.main - k) << 16;
   const Rec m = rec_of(run.main), own = rec_of(k);
-  for (int j = 0; j < kRecWords; ++j) f.w[kPure * kPureWords + j] = m.w[j];
-  for (uint32_t j = 0; j < (uint32_t)kFusedWords / 4u; ++j)
-    fused[(size_t)i * (kFusedWords / 4) + j] = make_uint4(f.w[4 * j], f.w[4 * j + 1], f.w[4 * j + 2], f.w[4 * j + 3]);
+  for (int j = 0; j < kRecWords; ++j) f.w[kPureFirst * kPureWords + j] = m.w[j];
+  store_fused();
   for (uint32_t j = 0; j < (uint32_t)kRecWords / 4u; ++j)
     recs[(size_t)i * (kRecWords / 4) + j] = make_uint4(own.w[4 * j], own.w[4 * j + 1], own.w[4 * j + 2], own.w[4 * j + 3]);
 }
@@ -748,7 +753,8 @@ struct Lane {
   // push or LD (a16),SP next to it makes) goes through write8.  x is a
   // 16-bit address.
   __device__ static bool plain_ram(uint32_t x) {
-    return (((0x3300u >> (x >> 12)) & 1u) != 0u) | (x - 0xFF80u < 0x7Fu);
+    // 8000-9FFF and C000-DFFF: bit 15 set, bit 13 clear
+    return ((x & 0xA000u) == 0x8000u) | (x - 0xFF80u < 0x7Fu);
   }
   __device__ static bool plain_store(uint32_t x) { return plain_ram(x) | (x == 0xFF00u); }
   // The instruction's bus writes, in order (n = 0, 1 or 2).  When both are
@@ -1317,7 +1323,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   // record of the instruction at pc, with the pure instructions that run
   // before it (the debug variants run every instruction alone)
   Rec rec{};
-  uint32_t pure[kPure * kPureWords];
+  uint32_t pure[kPureFirst * kPureWords];
+  const uint4* cur = fused;  // that record
   pure[7] = 0;
   // 0xFF once something has made the loaded record stale
   uint32_t stale = 0xFFu;
@@ -1340,15 +1347,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
   auto load_rec = [&](uint32_t i) {
     if (kDbg) return;
     stale = 0;
-    const uint4* p = fused + (size_t)i * (kFusedWords / 4);
-    ld_words(p, pure, kPure * kPureWords / 4);
-    ld_words(p + kPure * kPureWords / 4, rec.w, kRecWords / 4);
+    cur = fused + (size_t)i * (kFusedStride / 4);
+    ld_words(cur, pure, kPureFirst * kPureWords / 4);
+    ld_words(cur + kPureFirst * kPureWords / 4, rec.w, kRecWords / 4);
   };
   // no pure instruction ahead of the record
   auto clear_pure = [&]() {
     constexpr PureWords none = no_pure();
 #pragma unroll
-    for (uint32_t j = 0; j < kPure * kPureWords; ++j) pure[j] = none.w[j % kPureWords];
+    for (uint32_t j = 0; j < kPureFirst * kPureWords; ++j) pure[j] = none.w[j % kPureWords];
+    cur = fused + (size_t)L.no_rec * (kFusedStride / 4);
   };
 
   // Block copies of the copy-loop fast-forward (bytes cp_src[j * cp_stride]
@@ -1441,8 +1449,21 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       }
       uint32_t sph = L.sp << 16;
       if (!kDbg) {
-        exec_pure(pure, L.w0, L.w1, sph);
-        exec_pure(pure + kPureWords, L.w0, L.w1, sph);
+        const auto first = [&]() {
+          exec_pure(pure, L.w0, L.w1, sph);
+          exec_pure(pure + kPureWords, L.w0, L.w1, sph);
+        };
+        // the third and fourth sit in the record's second line, which a pass
+        // without them does not touch; the first two cover its latency
+        if (__ballot(pure[7] >= (kPureFirst + 1u) << 24) != 0u) {
+          uint32_t more[(kPure - kPureFirst) * kPureWords];
+          ld_words(cur + (kPureFirst * kPureWords + kRecWords) / 4, more, (kPure - kPureFirst) * kPureWords / 4);
+          first();
+          exec_pure(more, L.w0, L.w1, sph);
+          exec_pure(more + kPureWords, L.w0, L.w1, sph);
+        } else {
+          first();
+        }
         pc = (pc + (pure[kPureWords + 7] >> 16)) & 0xFFFFu;
         pc_before = pc;
         ninstr += pure[7] >> 24;
@@ -1459,7 +1480,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       ExecIn in;
       in.w0 = L.w0;
       in.w1 = L.w1;
-      in.x1 = bit_select(0xFFFF0000u, sph, pc);
+      in.x1 = bit_select<0xFFFF0000u>(sph, pc);
       in.ra = operand_address(rec, L.w0, L.w1, in.x1);
 
       // ---- bus reads ------------------------------------------------------------

@@ -39,6 +39,8 @@ static inline uint32_t sbfe(uint32_t v, uint32_t off, uint32_t width) {
 }
 template <int pos>
 static inline uint32_t bit_mask(uint32_t w) { return 0u - ((w >> pos) & 1u); }
+template <uint32_t m>
+static inline uint32_t bit_select(uint32_t a, uint32_t b) { return (a & m) | (b & ~m); }
 static inline uint32_t add_u16x2(uint32_t a, uint32_t b) {
   return ((a + b) & 0xFFFFu) | (((a >> 16) + (b >> 16)) << 16);
 }

@@ -352,8 +352,8 @@ def test_pure_datapath_matches_datapath(harness, seed):
 
 def test_fused_runs(harness):
     """Runs end at an instruction that is not pure, at the window's end, at a
-    jump out of the window or into its first 256 bytes, after two."""
-    out = _arr(5)
+    jump out of the window or into its first 256 bytes, after four."""
+    out = _arr(7)
 
     def run(code, at=0x200, lo=0, end=0x3FFE, abs_ok=1, size=0x8000):
         img = bytearray([0x76]) * size
@@ -364,7 +364,8 @@ def test_fused_runs(harness):
 
     assert run({0x200: b"\x76"}) == (0, 0, 0x200)
     assert run({0x200: b"\x78\x34"}) == (1, 4, 0x201, 0x200)
-    assert run({0x200: b"\x78\x01\x34\x12\x04"}) == (2, 16, 0x204, 0x200, 0x201)
+    assert run({0x200: b"\x78\x01\x34\x12\x04"}) == (3, 20, 0x205, 0x200, 0x201, 0x204)
+    assert run({0x200: b"\x78" * 6}) == (4, 16, 0x204, 0x200, 0x201, 0x202, 0x203)
     assert run({0x200: b"\xcb\x37\xcb\x36"}) == (1, 8, 0x202, 0x200)
     # the instruction after the run must have a record too
     assert run({0x3FFC: b"\x78\x78\x78"}, at=0x3FFC) == (1, 4, 0x3FFD, 0x3FFC)

@@ -1400,6 +1400,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
     }
   };
 
+  // Value of ninstr at the last HALT reached (hold, below).
+  uint32_t halt_at = 0;
+
   // One exit: the frame count reached or the env trapped (a trap freezes
   // the env for the rest of the launch, misc.py:42-56).
   while ((L.frames_done < frames) & (trap == 0)) {
@@ -1544,6 +1547,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
       // (a wave-uniform test, so that the copy below runs with every lane
       // that is executing an instruction)
       if (__builtin_expect(__ballot(o.misc != 0u) != 0u, 0)) {
+        const uint64_t act = __ballot(true);
         if (o.misc != 0u) {  // DI EI RETI HALT DAA, illegal opcodes, poll/copy loops
           count_pure();
           L.settle();  // the fast-forwards start from the PPU and timer state
@@ -1552,7 +1556,27 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
             L.ime_delay = 0;
           }
           if (o.misc & kMiscDaa) L.w1 = exec_daa(in.w1);
-          if (o.misc & kMiscHalt) L.halted = 1;
+          if (o.misc & kMiscHalt) {
+            // A lane that comes to HALT while others of its wavefront run
+            // holds for one pass: HALT runs once more, this one taking no
+            // cycles and not counting.  Fused runs break at each lane's own
+            // events, so that lanes of one short interrupt loop fall a pass
+            // out of step and each then pays the halted step, the interrupt
+            // and the rare blocks by itself; held, they halt and wake
+            // together (ROM-only loop of 40 instructions a wake, 16,384 /
+            // 131,072 envs frameskip 4: 762 / 991 us without, 520 / 690 with;
+            // 90 a wake, 131,072 envs: 1,665 / 1,315).  Only within 96
+            // instructions of the last HALT: after longer programs the others
+            // are rarely a pass away (MBC1, every program of its own length,
+            // 8,192 envs frameskip 4: 4.85 ms without, 4.93 with, 5.09
+            // with no bound).
+            const bool hold = !kDbg & (act != __ballot(true)) & (ninstr - halt_at - 1u < 96u) & (L.budget > 4);
+            halt_at = ninstr;
+            L.halted = hold ? 0u : 1u;
+            npc = hold ? pc : npc;
+            cycles = hold ? 0 : cycles;
+            ninstr -= hold ? 1u : 0u;
+          }
           // the step's interrupt check services or wakes on a pending request
           if (((L.ime | L.halted) != 0u) & ((L.ie & L.ifr & 0x1Fu) != 0u)) L.budget = 0;
           if (o.misc & kMiscTrap) {  // misc.py:42-56: freeze the env, pc unchanged
@@ -1697,13 +1721,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
             L.write8((L.sp - k) & 0xFFFFu, k == 1 ? ret >> 8 : ret & 0xFFu);
           L.sp = (L.sp - 2u) & 0xFFFFu;
           L.pc = 0x40u + 8u * (uint32_t)__builtin_ctz(bit);
-          stale = 0xFFu;
+          // (marked stale instead, the vector's jump ran in a pass alone,
+          // behind a load nothing covers: 1-2% of the interrupt-driven carts)
+          load_rec(L.next_rec(L.pc));
           svc = 20;
           L.timer_tick(20);
           lcdc_now = L.ppu_advance(20);
         } else if (hiter) {
           L.pc = (L.pc + 1u) & 0xFFFFu;  // IME=0 wake skips a byte
-          stale = 0xFFu;
+          load_rec(L.next_rec(L.pc));
         }
       }
       if (__builtin_expect(L.map_changed != 0u, 0)) {
@@ -1719,6 +1745,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void s
         // LCD toggles and frame ends (cpu_step_builder.py frame loop)
         instr += ninstr;
         cyc += ncyc;
+        halt_at -= ninstr;
         ninstr = 0;
         ncyc = 0;
         if (lcdc_prev && !(lcdc_now & 0x80u)) {

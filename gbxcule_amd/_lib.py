@@ -35,7 +35,9 @@ BUF_MEM, BUF_PIX, BUF_PIX_PACKED, BUF_OBS, BUF_REWARD, BUF_ACTIONS, BUF_CART_RAM
     INFO_OBS_DIM,
     INFO_CART_RAM_STRIDE,
     INFO_STEP_LANES,
-) = range(10)
+    INFO_STEP_THREADS,
+    INFO_STEP_WAVES,
+) = range(12)
 
 # Every symbol the header declares, with its ctypes signature.
 _vp, _i32, _i64 = ctypes.c_void_p, ctypes.c_int32, ctypes.c_int64

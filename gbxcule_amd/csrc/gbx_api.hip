@@ -201,6 +201,16 @@ int choose_step_lanes(int n, int kind, int cus) {
   }
   return kind != MBC_ROM_ONLY && (n + 7) / 8 <= cus ? 8 : kEnvBlock;
 }
+// Wavefronts per SIMD to build the step kernel for.  At two it holds what a
+// pass needs in about 200 VGPRs; at three it has 168 and spills up to 38 of
+// them, which is the lesser evil where the 64-env blocks are more than two to a
+// SIMD (131,072 envs) but no more than three, and two would leave a second
+// round of wavefronts behind the first.  Frameskip 4, 147,456 / 196,608 envs:
+// random code 34.7 / 40.5 ms at two, 24.9 / 32.2 at three; PPU cart frameskip
+// 24 714 / 751 us and 583 / 591; MBC1 frameskip 1 2,879 / 2,957 and 2,209 /
+// 2,512.  Past that both need as many rounds, or the third wavefront no longer
+// pays (262,144 envs: 42.3 and 51.7 ms, 327,680: 58.7 and 61.0).
+int choose_step_waves(int blocks, int cus) { return blocks > 2 * 4 * cus && blocks <= 3 * 4 * cus ? 3 : 2; }
 int cu_count() {
   int dev = 0, x = 0;
   if (hipGetDevice(&dev) == hipSuccess &&
@@ -262,6 +272,7 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   // against 9.3 / 9.4; level from 65,536 on, and 8.8 against 8.0 at 16,384).
   s.step_threads = s.step_lanes == kEnvBlock && kind != MBC_ROM_ONLY && ram_bytes > 0 && s.npad / kEnvBlock > cus
                        ? 4 * kEnvBlock : s.step_lanes;
+  s.step_waves = choose_step_waves(s.npad / kEnvBlock, cus);
   const size_t np = (size_t)s.npad;
   hipError_t e = hipSuccess;
   auto A = [&](hipError_t r) {
@@ -762,6 +773,8 @@ int gbx_info(gbx_ctx* ctx, int32_t key, int64_t* out) {
     case GBX_INFO_OBS_DIM: *out = s.obs_dim; break;
     case GBX_INFO_CART_RAM_STRIDE: *out = s.cram_stride; break;
     case GBX_INFO_STEP_LANES: *out = s.step_lanes; break;
+    case GBX_INFO_STEP_THREADS: *out = s.step_threads; break;
+    case GBX_INFO_STEP_WAVES: *out = s.step_waves; break;
     default: return fail(GBX_E_INVALID, "unknown info key");
   }
   return GBX_OK;

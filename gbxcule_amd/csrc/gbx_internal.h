@@ -97,6 +97,7 @@ struct DevState {
   int rom_banks, rom_mask, ram_banks, ram_bytes, cram_stride, mbc_kind;
   int step_lanes;       // envs per step-kernel wavefront: 64, 32, 16, 8 or 4
   int step_threads;     // threads of its workgroups: step_lanes, or 256
+  int step_waves;       // wavefronts per SIMD the step kernel is built for: 2 or 3
   int64_t rom_len;
   int64_t no_rec;       // bytes of the ROM buffer, the fused record that serves no pc
 };

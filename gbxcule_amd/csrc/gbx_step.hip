@@ -1210,13 +1210,11 @@ struct Lane {
 // ---------------------------------------------------------------------------
 // The kernel
 // ---------------------------------------------------------------------------
-// One variant per cartridge kind (kMbc), per debug mode (kDbg) and, for
-// ROM-only carts, per declared RAM (kCram): the cartridge code of other
-// kinds and every debug check compile out.  Built for two wavefronts per SIMD
-// (256 VGPRs, about 200 used): 131,072 envs in 64-lane wavefronts are two per
-// SIMD.
-template <int kMbc, bool kDbg, bool kCram = true>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void step_kernel(DevState s, StepArgs args) {
+// One variant per cartridge kind (kMbc), per debug mode (kDbg), per declared
+// RAM (kCram) and per wavefronts per SIMD (kWaves, choose_step_waves): the
+// cartridge code of other kinds and every debug check compile out.
+template <int kMbc, bool kDbg, bool kCram = true, int kWaves = 2>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void step_kernel(DevState s, StepArgs args) {
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (uint32_t)s.n) return;
   Lane L{s};
@@ -1880,26 +1878,30 @@ hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st) {
   const int blocks = (s.n + threads - 1) / threads;
   const bool dbg = a.dbg_rst38 || a.dbg_trap_pc || a.dbg_max_instr > 0 || a.dbg_watch;
   const dim3 g(blocks), b(threads);
-  const bool rom_ram = s.mbc_kind == MBC_ROM_ONLY && s.ram_banks > 0;
+  // (the variants without cartridge RAM have no store path for it; the debug
+  // variants of MBC carts keep the general one)
+  const bool ram = s.ram_banks > 0, three = s.step_waves == 3;
+  const auto run = [&](auto kernel2, auto kernel3) {
+    if (three) hipLaunchKernelGGL(kernel3, g, b, 0, st, s, a);
+    else hipLaunchKernelGGL(kernel2, g, b, 0, st, s, a);
+  };
   switch (s.mbc_kind * 2 + (dbg ? 1 : 0)) {
     case MBC_ROM_ONLY * 2:
-      if (rom_ram) hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, false, true>), g, b, 0, st, s, a);
-      else hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, false, false>), g, b, 0, st, s, a);
+      if (ram) run(step_kernel<MBC_ROM_ONLY, false, true, 2>, step_kernel<MBC_ROM_ONLY, false, true, 3>);
+      else run(step_kernel<MBC_ROM_ONLY, false, false, 2>, step_kernel<MBC_ROM_ONLY, false, false, 3>);
       break;
     case MBC_ROM_ONLY * 2 + 1:
-      if (rom_ram) hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, true>), g, b, 0, st, s, a);
+      if (ram) hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, true>), g, b, 0, st, s, a);
       else hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, false>), g, b, 0, st, s, a);
       break;
-    // (an MBC cart without RAM gets the variant whose store path has no
-    // cartridge RAM; the debug variants keep the general one)
     case MBC_MBC1 * 2:
-      if (s.ram_banks > 0) hipLaunchKernelGGL((step_kernel<MBC_MBC1, false, true>), g, b, 0, st, s, a);
-      else hipLaunchKernelGGL((step_kernel<MBC_MBC1, false, false>), g, b, 0, st, s, a);
+      if (ram) run(step_kernel<MBC_MBC1, false, true, 2>, step_kernel<MBC_MBC1, false, true, 3>);
+      else run(step_kernel<MBC_MBC1, false, false, 2>, step_kernel<MBC_MBC1, false, false, 3>);
       break;
     case MBC_MBC1 * 2 + 1: hipLaunchKernelGGL((step_kernel<MBC_MBC1, true>), g, b, 0, st, s, a); break;
     case MBC_MBC3 * 2:
-      if (s.ram_banks > 0) hipLaunchKernelGGL((step_kernel<MBC_MBC3, false, true>), g, b, 0, st, s, a);
-      else hipLaunchKernelGGL((step_kernel<MBC_MBC3, false, false>), g, b, 0, st, s, a);
+      if (ram) run(step_kernel<MBC_MBC3, false, true, 2>, step_kernel<MBC_MBC3, false, true, 3>);
+      else run(step_kernel<MBC_MBC3, false, false, 2>, step_kernel<MBC_MBC3, false, false, 3>);
       break;
     default: hipLaunchKernelGGL((step_kernel<MBC_MBC3, true>), g, b, 0, st, s, a); break;
   }

@@ -1,10 +1,11 @@
 """Step launches of every shape the env count and the cart choose: an env's
 state does not depend on the wavefront or workgroup it runs in.
 
-70 envs (checked against the oracle elsewhere) give the state hash of each of
-70 action sequences; larger counts repeat the sequences and must repeat the
-hashes, at counts on both sides of the rule's edges and with a partial last
-block and workgroup.
+70 envs (checked against the oracle elsewhere) give the state hash, cartridge
+RAM and serial bytes of each of 70 action sequences; larger counts repeat the
+sequences and must repeat these, at counts on both sides of the rules' edges
+(which follow the device's CU count) and with a partial last block and
+workgroup.
 """
 
 from __future__ import annotations
@@ -18,43 +19,86 @@ from .conftest import require_gpu
 
 pytestmark = pytest.mark.gpu
 
-BASE, STEPS = 70, 6
+BASE = 70
 
 
-def _hashes(rom, boot, n):
+def _state(rom, boot, n, steps):
+    """Hash of every env; cartridge RAM and serial bytes of the first and last
+    BASE envs; (lanes, threads, wavefronts per SIMD) of the launches."""
     import torch
 
+    from gbxcule_amd import _lib
     from gbxcule_amd.backend import HipVecBackend
 
     dut = HipVecBackend(rom, num_envs=n, frames_per_step=2, release_after_frames=1, stage="emulate_only", bootrom=boot)
     try:
         dut.reset(seed=0)
-        for k in range(STEPS):
+        for k in range(steps):
             act = np.resize(seeded_actions(7, k, BASE), n)
             dut.step_torch(torch.from_numpy(act).cuda())
-        return dut.state_hash_torch().cpu().numpy(), dut.step_lanes
+        shape = tuple(dut._info(k) for k in (_lib.INFO_STEP_LANES, _lib.INFO_STEP_THREADS, _lib.INFO_STEP_WAVES))
+        serial = dut.export_serial()
+        ends = [(0, min(BASE, n)), (max(0, n - BASE), n)]
+        return (
+            dut.state_hash_torch().cpu().numpy(),
+            [(lo, dut.export_cart_ram(lo, hi), serial[lo:hi]) for lo, hi in ends],
+            shape,
+        )
     finally:
         dut.close()
 
 
+def _same_for_every_shape(rom, boot, n, steps=6):
+    want, ((_, ram, serial), _), _ = _state(rom, boot, BASE, steps)
+    got, ends, shape = _state(rom, boot, n, steps)
+    np.testing.assert_array_equal(got, np.resize(want, n))
+    for lo, end_ram, end_serial in ends:
+        rows = (lo + np.arange(len(end_ram))) % BASE
+        np.testing.assert_array_equal(end_ram, ram[rows])
+        np.testing.assert_array_equal(end_serial, serial[rows])
+    return shape
+
+
+def _cus():
+    import torch
+
+    return torch.cuda.get_device_properties(0).multi_processor_count
+
+
 @pytest.mark.parametrize(
-    ("cart", "n", "lanes"),
+    ("cart", "count", "shape"),
     [
-        ("c1", 1, 64),
-        ("c2", 65, 64),
-        ("c2", 5003, 64),
-        ("c4", 63, 8),
-        ("c4", 2048, 8),
-        ("c4", 2049, 64),
-        ("c4m3", 2047, 8),
-        ("c4m3", 2049, 64),
-        ("c4m3", 16384, 64),  # one wavefront a workgroup
-        ("c4m3", 16449, 64),  # four, the last workgroup with two
+        ("c1", lambda cus: 1, (64, 64, 2)),
+        ("c2", lambda cus: 65, (64, 64, 2)),
+        ("c2", lambda cus: 5003, (64, 64, 2)),
+        ("c4", lambda cus: 63, (8, 8, 2)),
+        ("c4", lambda cus: 8 * cus, (8, 8, 2)),
+        ("c4", lambda cus: 8 * cus + 1, (64, 64, 2)),
+        ("c4m3", lambda cus: 8 * cus - 1, (8, 8, 2)),
+        ("c4m3", lambda cus: 8 * cus + 1, (64, 64, 2)),
+        # one wavefront a workgroup; four, the last workgroup with two
+        ("c4m3", lambda cus: 64 * cus, (64, 64, 2)),
+        ("c4m3", lambda cus: 64 * cus + 65, (64, 256, 2)),
     ],
 )
-def test_state_is_independent_of_the_launch_shape(carts, bootstub, cart, n, lanes):
+def test_state_is_independent_of_the_launch_shape(carts, bootstub, cart, count, shape):
     require_gpu()
-    want, _ = _hashes(carts[cart], bootstub, BASE)
-    got, got_lanes = _hashes(carts[cart], bootstub, n)
-    assert got_lanes == lanes
-    np.testing.assert_array_equal(got, np.resize(want, n))
+    assert _same_for_every_shape(carts[cart], bootstub, count(_cus())) == shape
+
+
+@pytest.mark.parametrize("cart", ["c2", "c4", "c4m3"])
+@pytest.mark.parametrize(
+    ("count", "waves"),
+    [
+        (lambda cus: 64 * 8 * cus, 2),
+        (lambda cus: 64 * 8 * cus + 1, 3),
+        (lambda cus: 64 * 12 * cus, 3),
+        (lambda cus: 64 * 12 * cus + 1, 2),
+    ],
+)
+def test_wavefronts_per_simd(carts, bootstub, cart, count, waves):
+    """Two wavefronts per SIMD up to 512 envs a CU, three to 768, then two."""
+    require_gpu()
+    n = count(_cus())
+    threads = 256 if cart == "c4m3" else 64
+    assert _same_for_every_shape(carts[cart], bootstub, n, steps=3) == (64, threads, waves)

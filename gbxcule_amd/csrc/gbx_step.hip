@@ -1213,7 +1213,7 @@ struct Lane {
 // One variant per cartridge kind (kMbc), per debug mode (kDbg), per declared
 // RAM (kCram) and per wavefronts per SIMD (kWaves, choose_step_waves): the
 // cartridge code of other kinds and every debug check compile out.
-template <int kMbc, bool kDbg, bool kCram = true, int kWaves = 2>
+template <int kMbc, bool kDbg, bool kCram, int kWaves>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) void step_kernel(DevState s, StepArgs args) {
   const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (uint32_t)s.n) return;
@@ -1342,8 +1342,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
     }
   };
   auto load_single = [&](uint32_t i) { ld_words(recs + (size_t)i * (kRecWords / 4), rec.w, kRecWords / 4); };
-  auto load_rec = [&](uint32_t i) {
-    if (kDbg) return;
+  auto load_rec = [&](uint32_t p) {
+    const uint32_t i = L.next_rec(p);
+    if (kDbg) {
+      stale = L.rec_ok(p) ? 0u : 0xFFu;
+      load_single(stale == 0u ? i : 0u);
+      return;
+    }
     stale = 0;
     cur = fused + (size_t)i * (kFusedStride / 4);
     ld_words(cur, pure, kPureFirst * kPureWords / 4);
@@ -1438,7 +1443,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
       // no record, or an event within the pure instructions (there is none
       // to run when cp is 0): the instruction at pc alone
       cp = max(ubfe(pure[7], 16, 8), stale);
-      const bool single = kDbg | ((int)cp >= min(max(L.budget, 1), 0xFF));
+      const bool single = (int)cp >= min(max(L.budget, 1), 0xFF);
       if (__builtin_expect(__ballot(single) != 0u, 0)) {
         if (single) {
           if (L.rec_ok(pc)) load_single(L.rec_index(pc));
@@ -1646,7 +1651,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
       }
       L.pc = npc;
       // fetch the next record while the writes, timer and PPU run
-      load_rec(L.next_rec(npc));
+      load_rec(npc);
       }
     } else {
       L.settle();
@@ -1721,13 +1726,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
           L.pc = 0x40u + 8u * (uint32_t)__builtin_ctz(bit);
           // (marked stale instead, the vector's jump ran in a pass alone,
           // behind a load nothing covers: 1-2% of the interrupt-driven carts)
-          load_rec(L.next_rec(L.pc));
+          load_rec(L.pc);
           svc = 20;
           L.timer_tick(20);
           lcdc_now = L.ppu_advance(20);
         } else if (hiter) {
           L.pc = (L.pc + 1u) & 0xFFFFu;  // IME=0 wake skips a byte
-          load_rec(L.next_rec(L.pc));
+          load_rec(L.pc);
         }
       }
       if (__builtin_expect(L.map_changed != 0u, 0)) {
@@ -1879,7 +1884,8 @@ hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st) {
   const bool dbg = a.dbg_rst38 || a.dbg_trap_pc || a.dbg_max_instr > 0 || a.dbg_watch;
   const dim3 g(blocks), b(threads);
   // (the variants without cartridge RAM have no store path for it; the debug
-  // variants of MBC carts keep the general one)
+  // variants of MBC carts keep the general one, and all of them, without the
+  // register-only instructions, fit three wavefronts per SIMD)
   const bool ram = s.ram_banks > 0, three = s.step_waves == 3;
   const auto run = [&](auto kernel2, auto kernel3) {
     if (three) hipLaunchKernelGGL(kernel3, g, b, 0, st, s, a);
@@ -1891,19 +1897,19 @@ hipError_t launch_step(const DevState& s, const StepArgs& a, hipStream_t st) {
       else run(step_kernel<MBC_ROM_ONLY, false, false, 2>, step_kernel<MBC_ROM_ONLY, false, false, 3>);
       break;
     case MBC_ROM_ONLY * 2 + 1:
-      if (ram) hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, true>), g, b, 0, st, s, a);
-      else hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, false>), g, b, 0, st, s, a);
+      if (ram) hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, true, 3>), g, b, 0, st, s, a);
+      else hipLaunchKernelGGL((step_kernel<MBC_ROM_ONLY, true, false, 3>), g, b, 0, st, s, a);
       break;
     case MBC_MBC1 * 2:
       if (ram) run(step_kernel<MBC_MBC1, false, true, 2>, step_kernel<MBC_MBC1, false, true, 3>);
       else run(step_kernel<MBC_MBC1, false, false, 2>, step_kernel<MBC_MBC1, false, false, 3>);
       break;
-    case MBC_MBC1 * 2 + 1: hipLaunchKernelGGL((step_kernel<MBC_MBC1, true>), g, b, 0, st, s, a); break;
+    case MBC_MBC1 * 2 + 1: hipLaunchKernelGGL((step_kernel<MBC_MBC1, true, true, 3>), g, b, 0, st, s, a); break;
     case MBC_MBC3 * 2:
       if (ram) run(step_kernel<MBC_MBC3, false, true, 2>, step_kernel<MBC_MBC3, false, true, 3>);
       else run(step_kernel<MBC_MBC3, false, false, 2>, step_kernel<MBC_MBC3, false, false, 3>);
       break;
-    default: hipLaunchKernelGGL((step_kernel<MBC_MBC3, true>), g, b, 0, st, s, a); break;
+    default: hipLaunchKernelGGL((step_kernel<MBC_MBC3, true, true, 3>), g, b, 0, st, s, a); break;
   }
   return hipGetLastError();
 }

@@ -519,7 +519,7 @@ int gbx_export_scalars(gbx_ctx* ctx, int32_t env, int64_t* scalars) {
 int gbx_packed_l1(const uint8_t* obs_dev, int64_t obs_stride, const uint8_t* goal_dev, int64_t goal_stride, int64_t n,
                   int64_t bytes, float scale, float* out_dev, void* stream) {
   // (a frame's sum, at most 12 per byte, stays in 32 bits)
-  if (n < 0 || bytes < 0 || bytes > (1 << 26) || n > (int64_t)INT32_MAX * 4)
+  if (n < 0 || bytes < 0 || bytes > (1 << 26))
     return fail(GBX_E_INVALID, "frame count or size out of range");
   if (n == 0) return GBX_OK;
   if (!out_dev || (bytes > 0 && (!obs_dev || !goal_dev))) return fail(GBX_E_INVALID, "frames or output NULL");

@@ -1,6 +1,7 @@
 // gbx_aux.hip -- kernels around the step: power-on fill, the 2x-downsampled
 // snapshot renderer, reset snapshot / masked restore, RAM-sense gather, state
 // hash, and the layout converters behind the export/import helpers.
+#include <algorithm>
 #include <type_traits>
 #include <utility>
 
@@ -940,19 +941,20 @@ template <typename W>
 __global__ __launch_bounds__(64 * kL1Waves) void packed_l1_kernel(const uint8_t* obs, int64_t obs_stride,
                                                                   const uint8_t* goal, int64_t goal_stride, int64_t n,
                                                                   uint32_t words, float scale, float* out) {
-  const int64_t i = (int64_t)blockIdx.x * kL1Waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (i >= n) return;
   const uint32_t l = threadIdx.x & 63u;
-  const W* a = reinterpret_cast<const W*>(obs + i * obs_stride);
-  const W* b = reinterpret_cast<const W*>(goal + i * goal_stride);
-  uint32_t acc = 0;
-  for (uint32_t w = l; w < words; w += 64u) {
-    if constexpr (sizeof(W) == 1) acc = shade_sad((uint32_t)a[w], (uint32_t)b[w], acc);
-    else acc = shade_sad(a[w], b[w], acc);
-  }
+  int64_t i = (int64_t)blockIdx.x * kL1Waves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  for (; i < n; i += (int64_t)gridDim.x * kL1Waves) {
+    const W* a = reinterpret_cast<const W*>(obs + i * obs_stride);
+    const W* b = reinterpret_cast<const W*>(goal + i * goal_stride);
+    uint32_t acc = 0;
+    for (uint32_t w = l; w < words; w += 64u) {
+      if constexpr (sizeof(W) == 1) acc = shade_sad((uint32_t)a[w], (uint32_t)b[w], acc);
+      else acc = shade_sad(a[w], b[w], acc);
+    }
 #pragma unroll
-  for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m, 64);
-  if (l == 0u) out[i] = (float)(int32_t)acc * scale;
+    for (int m = 32; m > 0; m >>= 1) acc += __shfl_xor(acc, m, 64);
+    if (l == 0u) out[i] = (float)(int32_t)acc * scale;
+  }
 }
 
 // Layout converters for the synchronous export/import helpers.
@@ -1140,7 +1142,9 @@ hipError_t launch_hash(const DevState& s, const HashTable& k, uint64_t* out, hip
 
 hipError_t launch_packed_l1(const uint8_t* obs, int64_t obs_stride, const uint8_t* goal, int64_t goal_stride,
                             int64_t n, int64_t bytes, float scale, float* out, hipStream_t st) {
-  const dim3 g((unsigned)((n + kL1Waves - 1) / kL1Waves)), b(64 * kL1Waves);
+  // (a grid has fewer than 2^32 threads; beyond 2^24 frames a wavefront takes
+  // several)
+  const dim3 g((unsigned)std::min<int64_t>((n + kL1Waves - 1) / kL1Waves, 1 << 22)), b(64 * kL1Waves);
   // 16 or 4 bytes a load where every frame starts and ends on that boundary,
   // else single bytes (odd frame widths, views at odd offsets)
   const uint64_t align = (uint64_t)(uintptr_t)obs | (uint64_t)(uintptr_t)goal | (uint64_t)obs_stride |

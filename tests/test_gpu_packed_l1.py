@@ -69,6 +69,20 @@ def test_all_shade_pairs_and_capture():
         assert torch.equal(out, packed_l1_distance(obs, goals))
 
 
+def test_more_frames_than_a_grid_has_wavefronts():
+    """2^26 + 3 one-byte frames: one wavefront each would be a grid of more
+    than 2^32 threads.  A frame's distance is that of its byte."""
+    require_gpu()
+    n = (1 << 26) + 3
+    gen = torch.Generator(device="cuda").manual_seed(9)
+    obs = torch.randint(0, 256, (n, 1, 1, 1), dtype=torch.uint8, device="cuda", generator=gen)
+    goal = torch.tensor([0xB4], dtype=torch.uint8, device="cuda").view(1, 1, 1, 1)
+    by_byte = packed_l1_distance(torch.arange(256, dtype=torch.uint8).view(256, 1, 1, 1), goal.cpu())
+    got = packed_l1_distance(obs, goal)
+    want = by_byte.cuda()[obs.view(-1).long()]
+    torch.testing.assert_close(got, want, rtol=2.4e-7, atol=0)
+
+
 def test_vmap_sees_torch_calls():
     require_gpu()
     gen = torch.Generator(device="cuda").manual_seed(5)

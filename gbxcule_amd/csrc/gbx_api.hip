@@ -148,10 +148,17 @@ hipError_t dalloc(T** p, size_t count) {
   return hipMalloc(reinterpret_cast<void**>(p), count * sizeof(T) > 0 ? count * sizeof(T) : 1);
 }
 
-// The ROM buffer, in 16 KiB windows: the ROM, one of 0xFF that an unmapped
-// ROM bank reads (open bus), and the banks that the window at 0000 can hold
-// (bank 0, and on an MBC1 cart banks 32, 64 and 96) with the boot image over
-// their first 256 bytes.
+// Bytes of a ROM that a window can hold: two banks without a bank controller,
+// 128 with one (7-bit bank numbers).  The records take 320 bytes for each:
+// 20 MiB for a 32 KiB cart, 340 MiB for 1 MiB and 660 MiB for 2 MiB and more.
+int64_t reachable_rom(int64_t rom_bytes, int kind) {
+  return std::min<int64_t>(rom_bytes, kind == MBC_ROM_ONLY ? 0x8000 : 128 * 0x4000);
+}
+
+// The ROM buffer, in 16 KiB windows: the reachable ROM, one of 0xFF that an
+// unmapped ROM bank reads (open bus), and the banks that the window at 0000
+// can hold (bank 0, and on an MBC1 cart banks 32, 64 and 96) with the boot
+// image over their first 256 bytes.
 std::vector<uint8_t> rom_buffer(const uint8_t* rom, int64_t rom_bytes, const uint8_t* boot, int kind) {
   std::vector<uint8_t> b(rom, rom + rom_bytes);
   b.resize(b.size() + 0x4000, 0xFF);
@@ -263,7 +270,7 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   s.ram_banks = ram_bytes / 0x2000;
   s.cram_stride = ram_bytes > 0 ? ram_bytes : 1;
   s.mbc_kind = kind;
-  s.rom_len = rom_bytes;
+  s.rom_len = reachable_rom(rom_bytes, kind);
   const int cus = cu_count();
   s.step_lanes = choose_step_lanes(num_envs, kind, cus);
   // One wavefront to a workgroup, except for carts with a bank controller and
@@ -294,7 +301,7 @@ int gbx_create(int32_t num_envs, const uint8_t* rom, int64_t rom_len, const uint
   uint8_t *drom = nullptr, *dboot = nullptr;
   Rec* drecs = nullptr;
   uint32_t* dfused = nullptr;
-  const std::vector<uint8_t> rombuf = rom_buffer(rom, rom_bytes, boot, kind);
+  const std::vector<uint8_t> rombuf = rom_buffer(rom, s.rom_len, boot, kind);
   s.no_rec = (int64_t)rombuf.size();
   A(dalloc(&drom, rombuf.size()));
   A(dalloc(&dboot, (size_t)0x100));

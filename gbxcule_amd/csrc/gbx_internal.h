@@ -87,8 +87,9 @@ struct DevState {
   uint8_t* pix_packed;  // [n][72][20]
   uint8_t* latches;     // [144][kLatchStride] env-0 scanline latches, one 16-byte entry per line
   uint8_t* frame_bg;    // [144][160] env-0 full-frame shades
-  // 16 KiB windows: the ROM; one of 0xFF (open bus); copies of the banks that
-  // window 0 can hold, with the boot image in their first 256 bytes
+  // 16 KiB windows: the ROM, as far as a bank number reaches; one of 0xFF
+  // (open bus); copies of the banks that window 0 can hold, with the boot image
+  // in their first 256 bytes
   const uint8_t* rom;
   const uint8_t* boot;
   const uint4* recs;        // pre-decoded instruction record per byte of the ROM buffer
@@ -98,7 +99,7 @@ struct DevState {
   int step_lanes;       // envs per step-kernel wavefront: 64, 32, 16, 8 or 4
   int step_threads;     // threads of its workgroups: step_lanes, or 256
   int step_waves;       // wavefronts per SIMD the step kernel is built for: 2 or 3
-  int64_t rom_len;
+  int64_t rom_len;      // of the ROM in the buffer: what its windows can reach
   int64_t no_rec;       // bytes of the ROM buffer, the fused record that serves no pc
 };
 

@@ -24,8 +24,10 @@ on one thread.
 from __future__ import annotations
 
 import argparse
+import hashlib
 import json
 import os
+import re
 import sys
 import time
 from dataclasses import replace
@@ -138,6 +140,28 @@ def profile_file(key: str, n: int, fs: int):
     return json.loads(f.read_text()) if f.exists() else None
 
 
+def step_kernel_hash() -> str:
+    """Hash of the step kernel's sources, comments and layout aside, and of
+    the flags they are compiled with."""
+    from gbxcule_amd.build import CSRC, DEVICE_FLAGS
+
+    h = hashlib.sha256(" ".join(DEVICE_FLAGS).encode())
+    for name in ("gbx_step.hip", "gbx_exec.h", "gbx_decode.h", "gbx_internal.h"):
+        text = re.sub(r"//[^\n]*|/\*.*?\*/", " ", (CSRC / name).read_text(), flags=re.S)
+        h.update(" ".join(text.split()).encode())
+    return h.hexdigest()[:16]
+
+
+def current_profile(key: str, res: dict):
+    """The rocprof summary of this workload shape if it is one of the kernel
+    as built and of the wavefronts this run launched, else None: counters of
+    another kernel say nothing about this run's time."""
+    prof = profile_file(key, res["num_envs"], res["frameskip"])
+    if prof is None or prof.get("kernel_hash") != step_kernel_hash():
+        return None
+    return prof if res.get("step_lanes", prof.get("step_lanes")) == prof.get("step_lanes") else None
+
+
 def time_workload(wl, steps: int, warmup: int, settle: int = 0) -> dict:
     """Run ``settle`` + ``warmup`` + ``steps`` steps of ``wl`` and time the
     last ``steps``."""
@@ -244,11 +268,12 @@ def time_workload(wl, steps: int, warmup: int, settle: int = 0) -> dict:
 
 def roofline(key: str, res: dict, data_b: float, instr_b: float) -> dict:
     """Step-kernel roofline: algorithmic bytes per launch over its measured
-    duration; rocprof traffic per launch where a committed summary exists."""
+    duration; rocprof traffic per launch where a committed summary of this
+    kernel exists."""
     n, fs, kernel_ms = res["num_envs"], res["frameskip"], res["step_kernel_ms"]
     bytes_per_env_step = STATE_BYTES + data_b
     achieved = n * bytes_per_env_step / (kernel_ms * 1e-3) / 1e9
-    prof = profile_file(key, n, fs)
+    prof = current_profile(key, res)
     out = {
         "bound": "hbm",
         "achieved": achieved,
@@ -269,9 +294,9 @@ def roofline(key: str, res: dict, data_b: float, instr_b: float) -> dict:
 
 def valu_object(key: str, res: dict):
     """VALU issue against the chip's peak: profiled wave-instructions per
-    launch (committed rocprof summary of the same workload) x 64 lanes over
+    launch (committed rocprof summary of this kernel and workload) x 64 lanes over
     this run's measured kernel time, plus the profiled active-lane fraction."""
-    prof = profile_file(key, res["num_envs"], res["frameskip"])
+    prof = current_profile(key, res)
     if not prof or not prof.get("valu_wave_insts_per_launch"):
         return None
     lane_ops = prof["valu_wave_insts_per_launch"] * 64 / (res["step_kernel_ms"] * 1e-3)

@@ -47,6 +47,38 @@ def test_timed_workloads_have_profile_summaries(key, n, fs):
     assert f"{n:,}" in text and "FETCH_SIZE" in text and "WRITE_SIZE" in text
 
 
+@pytest.mark.parametrize("key,n,fs", TIMED)
+def test_summaries_of_another_kernel_are_not_used(monkeypatch, key, n, fs):
+    prof = bench.profile_file(key, n, fs)
+    res = {"num_envs": n, "frameskip": fs, "step_kernel_ms": 1.0, "step_lanes": prof["step_lanes"]}
+    assert bench.current_profile(key, res) == prof
+    assert bench.roofline(key, res, 1.0, 1.0)["traffic"] == prof["bytes_per_launch"]
+    assert bench.valu_object(key, res) is not None
+    for other in ({**res, "step_lanes": 16}, res):
+        if other is res:
+            monkeypatch.setattr(bench, "step_kernel_hash", lambda: "0" * 16)
+        assert bench.current_profile(key, other) is None
+        assert bench.roofline(key, other, 1.0, 1.0)["traffic"] is None
+        assert bench.valu_object(key, other) is None
+
+
+def test_kernel_hash_follows_code_not_comments(monkeypatch, tmp_path):
+    from gbxcule_amd import build
+
+    names = ("gbx_step.hip", "gbx_exec.h", "gbx_decode.h", "gbx_internal.h")
+    for name in names:
+        (tmp_path / name).write_text((build.CSRC / name).read_text())
+    before = bench.step_kernel_hash()
+    monkeypatch.setattr(build, "CSRC", tmp_path)
+    assert bench.step_kernel_hash() == before
+    f = tmp_path / "gbx_exec.h"
+    text = f.read_text()
+    f.write_text("// a remark\n" + text + "\n/* and\nanother */\n")
+    assert bench.step_kernel_hash() == before
+    f.write_text(text + "constexpr int kOneMore = 1;\n")
+    assert bench.step_kernel_hash() != before
+
+
 def test_roofline_and_valu_objects():
     res = {"num_envs": 131_072, "frameskip": 24, "step_kernel_ms": 2.0}
     data_b = 10_000.0

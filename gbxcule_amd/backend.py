@@ -177,7 +177,7 @@ class HipVecBackend:
 
     @property
     def step_lanes(self) -> int:
-        """Envs per wavefront of the step kernel (64, 32, 16 or 8)."""
+        """Envs per wavefront of the step kernel (64, 32, 16, 8 or 4)."""
         return self._info(_lib.INFO_STEP_LANES)
 
     def _info(self, key: int) -> int:

@@ -196,10 +196,15 @@ int parse_header(const uint8_t* rom, int64_t rom_len, int* kind, int64_t* rom_by
 // and 16,384 envs are one wavefront per CU: random-code cart, frameskip 4, at
 // 8,192 / 16,384 / 32,768 envs 10.7 / 10.7 / 11.8 ms with 64 envs a wavefront,
 // 12.3 / 11.2 / 12.5 with 32, 18.0 / 11.4 / 15.9 with 16.  Carts with a bank
-// controller run interrupt and halt handling in which each lane delays the
-// others: while it still gives every CU at most one wavefront, 8 envs a
-// wavefront are faster (MBC1 at 64 / 2,048 envs 4.4 / 4.6 ms against 5.1 / 5.4
-// with 64; at 4,096 envs they are level).
+// controller may run another bank, another program, in each lane, and meet IO,
+// interrupts and HALT each at its own time: while it still gives every CU at
+// most one wavefront, 8 envs a wavefront are faster for those (random programs
+// in 31 banks, frameskip 4, at 64 / 512 / 2,048 envs: MBC1 4.3 / 4.6 / 4.6 ms
+// against 4.9 / 5.0 / 5.1 with 64, MBC3 6.3 / 6.8 / 7.0 against 7.6 / 7.8 /
+// 7.9), though not for a short loop that all lanes share (MBC1, 0.63 / 0.66 /
+// 0.66 ms against 0.56).  It is the banks that tell: the same interrupts and
+// HALT around one program without a bank controller run in 2.6 / 2.8 / 2.8 ms
+// with 8 and 2.7 with 64, a shared short loop in 0.60 / 0.62 / 0.62 and 0.53.
 // GBX_STEP_LANES=64|32|16|8|4 overrides the choice (for tuning sweeps).
 int choose_step_lanes(int n, int kind, int cus) {
   if (const char* v = getenv("GBX_STEP_LANES")) {

@@ -472,7 +472,7 @@ __host__ __device__ constexpr uint32_t poll_loop_len(const uint8_t* p, uint32_t 
   if ((j == 0x20u || j == 0x28u || j == 0x30u || j == 0x38u) && p[n + 3] == ((0x100u - (n + 4u)) & 0xFFu))
     return n + 4u;
   // (a JP target at or above 0x8000 is never the load's pc: records exist
-  // only for ROM and the boot image, and bit 31 of DW marks a copy loop)
+  // only for the windows below it, and bit 31 of DW marks a copy loop)
   if ((j == 0xC2u || j == 0xCAu || j == 0xD2u || j == 0xDAu) && avail >= n + 5u && p[n + 4] < 0x80u)
     return n + 5u;
   return 0;

@@ -20,7 +20,7 @@
 //    first line; the others cost a pass nothing where no lane has them.  With
 //    none / two / four, same launch shape for the last two: 16,384 envs
 //    frameskip 24 128.0 / 71.9 / 67.7 ms, 64 envs frameskip 4 29.7 / 13.9 /
-//    11.9 ms.  A pass whose register-only instructions would reach an event
+//    11.9 ms; a pass where no lane has any runs none.  A pass whose register-only instructions would reach an event
 //    (event_budget) runs the instruction at pc alone;
 //  * what an instruction computes without the bytes it reads (carry-in,
 //    branch, SP, write addresses) is pinned behind the issue of the read,
@@ -29,7 +29,7 @@
 //    byte permutes of the register file and the bus bytes selected by the
 //    record, with one shared adder, logic unit, shifter and 16-bit adder, so
 //    no lane waits for another lane's opcode class;
-//  * bus reads compute one address per lane (ROM window, boot image,
+//  * bus reads compute one address per lane (a window of the ROM buffer,
 //    cartridge RAM or the env's memory) and every lane loads its byte, with
 //    no branch around the load; only a second byte, IO side effects, MBC and
 //    cartridge-RAM writes take divergent branches;
@@ -270,9 +270,9 @@ struct Lane {
   // The byte the bus reads at A000 (cart_p) and the mask of the row offset
   // of an A000-BFFF address (cart_m): ~0 while a RAM bank is mapped; 0 while
   // an RTC register is (every address reads the low byte of its cartridge
-  // state slot) or nothing is (every address reads a byte of the 0xFF filler
-  // that follows the boot image in the ROM buffer, which is what disabled or
-  // absent cartridge RAM returns).
+  // state slot) or nothing is (every address reads a byte of the 0xFF window
+  // that follows the ROM in the ROM buffer, which is what disabled or absent
+  // cartridge RAM returns).
   const uint8_t* cart_p;
   uint32_t cart_m;
   int rtc_sub;
@@ -391,10 +391,10 @@ struct Lane {
     return x == 0xFF41u ? stat_val() : v;
   }
   __device__ static bool io_derived(uint32_t x) { return (x & 0xFFBAu) == 0xFF00u; }
-  // Flat address of the byte the bus returns at x (echo-folded): ROM window,
-  // boot image, or the 0xFF filler for an unmapped bank; cartridge RAM, the
-  // mapped RTC register, or the 0xFF filler for disabled or absent cartridge
-  // RAM; or the env's memory.
+  // Flat address of the byte the bus returns at x (echo-folded): a window of
+  // the ROM buffer (a bank, its copy under the boot image, or the 0xFF window
+  // for an unmapped bank); cartridge RAM, the mapped RTC register, or a byte of
+  // the 0xFF window for disabled or absent cartridge RAM; or the env's memory.
   __device__ const uint8_t* bus_ptr(uint32_t x) const {
     const bool rom = x < 0x8000u;
     const bool cart = x - 0xA000u < 0x2000u;
@@ -1236,7 +1236,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kWaves))) v
                     kCartStateStride * kEnvBlock * 4);
   const rsrc_t rcnt = make_rsrc(s.cnt + (size_t)blk * (2 * kEnvBlock), 2 * kEnvBlock * 8);
   const uint4* recs = in_vgpr(reinterpret_cast<const uint4*>(s.recs));    // 4 per record
-  const uint4* fused = in_vgpr(reinterpret_cast<const uint4*>(s.fused));  // 8 per fused record
+  const uint4* fused = in_vgpr(reinterpret_cast<const uint4*>(s.fused));  // 16 per fused record
 
   // ---- load (cpu_step_builder.py:930-967) ---------------------------------
   L.pc = (uint32_t)L.SC(F_PC) & 0xFFFFu;

@@ -1,7 +1,8 @@
-"""The goal-distance kernel against the torch form of the same function, which
-CPU tensors take: the same sums of whole numbers, one rounding each, then one
-multiplication by the 32-bit reciprocal where the CPU divides (so a relative
-difference of at most 2 units in the last place, 2.4e-7).  Forms: one goal and
+"""The goal-distance kernel against the torch form of the same function: on
+the GPU the same bits (the same sums of whole numbers, then a multiplication
+by the 32-bit reciprocal, as torch divides by a number there); on the CPU,
+which divides, a relative difference of at most 2 units in the last place,
+2.4e-7.  Forms: one goal and
 one per env, frame widths that allow 16-, 4- and 1-byte loads, views at odd
 offsets and with gaps between frames, and forms that stay with torch."""
 
@@ -18,8 +19,13 @@ pytestmark = pytest.mark.gpu
 
 
 def _check(obs, goal):
+    from gbxcule_amd.rl import packed
+
     want = packed_l1_distance(obs.cpu(), goal.cpu())
     got = packed_l1_distance(obs, goal)
+    with pytest.MonkeyPatch.context() as mp:
+        mp.setattr(packed, "_l1_kernel_operands", lambda *_: None)
+        assert torch.equal(got, packed_l1_distance(obs, goal))
     assert got.dtype is torch.float32 and got.shape == want.shape and got.device == obs.device
     torch.testing.assert_close(got.cpu(), want, rtol=2.4e-7, atol=0)
     if obs.shape[1] == 1:

@@ -13,7 +13,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from gbxcule_amd.carts.synth import seeded_actions
+from gbxcule_amd.carts.synth import finalize_rom, seeded_actions
 
 from .conftest import require_gpu
 
@@ -102,3 +102,54 @@ def test_wavefronts_per_simd(carts, bootstub, cart, count, waves):
     n = count(_cus())
     threads = 256 if cart == "c4m3" else 64
     assert _same_for_every_shape(carts[cart], bootstub, n, steps=3) == (64, threads, waves)
+
+
+# (cartridge type, ROM size code, RAM size code) over a cart's program: the
+# kernel variants that the carts themselves do not reach
+@pytest.mark.parametrize(
+    ("cart", "header"),
+    [
+        ("c3", None),
+        ("c2", (0x00, 0x00, 0x02)),
+        ("c4", (0x03, 0x04, 0x03)),
+        ("c4m3", (0x11, 0x04, 0x00)),
+    ],
+)
+def test_three_wavefronts_of_every_variant(carts, bootstub, cart, header):
+    """LY polls, block copies, and each cartridge kind with and without RAM."""
+    require_gpu()
+    rom = carts[cart]
+    if header is not None:
+        rom = finalize_rom(bytearray(rom), "GBXAMD", *header)
+    n = 64 * 8 * _cus() + 1
+    assert _same_for_every_shape(rom, bootstub, n, steps=12)[2] == 3
+
+
+def test_captured_step_of_three_wavefronts(carts, bootstub):
+    """A captured step, its variant's first launch, replayed between eager
+    work: the build for three wavefronts spills to scratch memory."""
+    require_gpu()
+    import torch
+
+    from gbxcule_amd.backend import HipVecBackend
+
+    n = 64 * 8 * _cus() + 1
+    act = torch.from_numpy(seeded_actions(7, 0, n)).cuda()
+    pair = [HipVecBackend(carts["c1"], num_envs=n, frames_per_step=1, release_after_frames=1, stage="emulate_only",
+                          bootrom=bootstub) for _ in range(2)]  # fmt: skip
+    try:
+        for be in pair:
+            be.reset(seed=0)
+        captured, eager = pair
+        graph = torch.cuda.CUDAGraph()
+        torch.cuda.synchronize()
+        with torch.cuda.graph(graph):
+            captured.step_torch(act)
+        for _ in range(3):
+            graph.replay()
+            eager.step_torch(act)
+            torch.cuda.synchronize()
+            assert torch.equal(captured.state_hash_torch(), eager.state_hash_torch())
+    finally:
+        for be in pair:
+            be.close()
